@@ -31,39 +31,31 @@ int launch_decode_wide(const uint16_t* x, int64_t m, int64_t x_stride, const lf_
                        bool exact, bool swiglu, bool withhold, void* stream);
 constexpr int64_t kDecodeMaxTokens = 64;
 
+double prefill_us(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu);
+
 // Whether the wide decode kernel (32 rows x 32 tokens per workgroup over the
-// whole K) serves M > 64 tokens faster than the prefill GEMM. Costs in us from
-// measured times on MI355X: a round of 256 wide workgroups takes about 4 us
-// per 4096 of K (its per-CU x and weight reads); a prefill round of 256 x 192
-// tiles about 85 us per 4096 of K.
-bool wide_cheaper(int64_t m, int64_t n, int64_t k) {
+// whole K) serves M > 64 tokens faster than the prefill GEMM (prefill_us):
+// a round of 256 wide workgroups takes 7.5 us per 4096 of K, 8.8 us with LoRA
+// (its per-CU x and weight reads; 256 tokens x 4096: 30 / 40 us against 56 /
+// 65 us on the prefill GEMM, 256 x 11008: 98 us against 67 us).
+bool wide_cheaper(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) {
   const int64_t cus = device_cus();
   const int64_t wide_groups = ((n / 32 + 7) / 8) * 8 * ((m + 31) / 32);
-  const double wide_us = double((wide_groups + cus - 1) / cus) * 4.0 * double(k) / 4096.0;
-  const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
-  const double prefill_us = double((tiles + cus - 1) / cus) * 85.0 * double(k) / 4096.0;
-  return wide_us < prefill_us;
+  const double wide_us = double((wide_groups + cus - 1) / cus) * (lora ? 8.8 : 7.5) * double(k) / 4096.0;
+  return wide_us < prefill_us(m, n, k, lora, swiglu);
 }
 
-// Whether M > 64 tokens are served faster by the decode kernel over 64-token
-// chunks than by one prefill launch. The prefill GEMM runs 256 x 192 tiles,
-// one workgroup per CU, so a call with fewer tiles than CUs leaves the rest
-// of the chip idle (c4: 256 tokens x 4096 features are 22 tiles on 256 CUs);
-// each decode chunk streams W again but uses every CU. Costs in us, from
-// measured times on MI355X: a decode launch of 64 tokens streams its weight
-// bytes (packed + fp32 scales) at about 0.8 TB/s, plus about 6 us with LoRA
-// (4096 x 4096: 11.9 us base only, 18.0 us with 32 rank-16 adapters); a
-// prefill round of tiles takes about 85 us per 4096 of K (c5: 1.81 rounds in
-// 189 us; c4: one round of 22 tiles in 77 us), plus about 20 us with LoRA.
-bool decode_chunks_cheaper(int64_t m, int64_t n, int64_t k, bool lora) {
+// Whether M > 64 tokens that the wide kernel does not take are served faster
+// by decode launches over 64-token chunks than by one prefill launch (few
+// tiles leave most of the chip idle; each decode chunk streams W again but
+// uses every CU). A decode launch of 64 tokens streams its weight bytes
+// (packed + fp32 scales) at about 0.8 TB/s, plus about 6 us with LoRA (4096 x
+// 4096: 11.9 us base only, 18.0 us with 32 rank-16 adapters).
+bool decode_chunks_cheaper(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) {
   const double weight_bytes = double(n) * double(k) * (0.5 + 4.0 / 64.0);
   const double chunk_us = (lora ? 6.0 : 0.0) + weight_bytes / 0.8e6;
   const int64_t chunks = (m + kDecodeMaxTokens - 1) / kDecodeMaxTokens;
-  const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
-  const int64_t cus = device_cus();
-  const int64_t rounds = (tiles + cus - 1) / cus;
-  const double prefill_us = double(rounds) * 85.0 * double(k) / 4096.0 + (lora ? 20.0 : 0.0);
-  return double(chunks) * chunk_us < prefill_us;
+  return double(chunks) * chunk_us < prefill_us(m, n, k, lora, swiglu);
 }
 // One decode launch of up to 64 tokens: the wide kernel for the batches and
 // shapes it takes (above 8 tokens, above 2 at N >= 8192, above 16 at
@@ -125,7 +117,7 @@ extern "C" int lf_nf4_lora_linear(const uint16_t* x, int64_t m, int64_t x_stride
   // unless the prefill GEMM is forced or cheaper, or the shape is outside the
   // kernel's range.
   if (lf::decode_wide_fits(m, n, k, lora) && !(flags & LF_PLAN_PREFILL) &&
-      (m <= lf::kDecodeMaxTokens || (flags & LF_PLAN_DECODE_CHUNKS) || lf::wide_cheaper(m, n, k)))
+      (m <= lf::kDecodeMaxTokens || (flags & LF_PLAN_DECODE_CHUNKS) || lf::wide_cheaper(m, n, k, lora != nullptr, swiglu)))
     return lf::launch_decode_wide(x, m, x_stride, w, bias, lora, y, y_stride, workspace, workspace_bytes, exact,
                                   swiglu, withhold, stream);
   if (m <= lf::kDecodeMaxTokens)
@@ -133,7 +125,7 @@ extern "C" int lf_nf4_lora_linear(const uint16_t* x, int64_t m, int64_t x_stride
                              withhold, stream);
   bool chunked = false;
   if (flags & LF_PLAN_DECODE_CHUNKS) chunked = true;
-  else if (!(flags & LF_PLAN_PREFILL)) chunked = lf::decode_chunks_cheaper(m, n, k, lora != nullptr);
+  else if (!(flags & LF_PLAN_PREFILL)) chunked = lf::decode_chunks_cheaper(m, n, k, lora != nullptr, swiglu);
   if (!chunked)
     return lf::launch_nf4_lora_prefill(x, m, x_stride, w, bias, lora, y, y_stride, workspace, workspace_bytes,
                                        swiglu, withhold, stream);

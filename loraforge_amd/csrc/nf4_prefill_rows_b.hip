@@ -1,0 +1,7 @@
+// Prefill GEMM instances (prefill_tile.h).
+#include "prefill_tile.h"
+
+namespace lf::prefill {
+template int launch_rows<6>(const PrefillParams&, int64_t, bool, bool, hipStream_t);
+template int launch_rows<2>(const PrefillParams&, int64_t, bool, bool, hipStream_t);
+}  // namespace lf::prefill
