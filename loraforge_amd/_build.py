@@ -21,6 +21,7 @@ ROOT = PACKAGE.parent
 CSRC = PACKAGE / "csrc"
 LIBDIR = PACKAGE / "_lib"
 LIBRARY = LIBDIR / "libloraforge_amd.so"
+BINDING = LIBDIR / "_binding.so"
 ARCH = "gfx950"
 
 HIP_FLAGS = [
@@ -93,6 +94,26 @@ def _compile(src: Path, obj: Path, verbose: bool) -> None:
         print("\n".join(messages), flush=True)
 
 
+def _compile_binding(verbose: bool) -> None:
+    """The operators' native call path (``csrc/host/binding.cpp``): host code against torch's headers."""
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    rocm = Path(hipcc()).resolve().parent.parent
+    tmp = BINDING.with_suffix(".so.tmp")
+    includes = [f"-I{p}" for p in (*include_paths(), sysconfig.get_paths()["include"], rocm / "include")]
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+           *includes, str(CSRC / "host" / "binding.cpp"), *(f"-L{p}" for p in library_paths()),
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-o", str(tmp)]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError("binding.cpp failed to compile:\n" + result.stderr)
+    os.replace(tmp, BINDING)
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
     """Compile every HIP source and link the library; returns its path."""
     objdir = LIBDIR / "obj"
@@ -101,7 +122,9 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     objs = [objdir / (s.stem + ".o") for s in srcs]
     workers = jobs or min(len(srcs), max(1, min(8, os.cpu_count() or 1)))
     with ThreadPoolExecutor(max_workers=workers) as pool:
+        binding = pool.submit(_compile_binding, verbose)
         list(pool.map(lambda pair: _compile(pair[0], pair[1], verbose), zip(srcs, objs)))
+        binding.result()
     tmp = LIBRARY.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     if verbose:

@@ -14,6 +14,7 @@ import threading
 from pathlib import Path
 
 LIBRARY = Path(__file__).resolve().parent / "_lib" / "libloraforge_amd.so"
+BINDING = LIBRARY.with_name("_binding.so")
 
 LF_OK = 0
 LF_EINVAL = 1
@@ -25,6 +26,14 @@ LF_PLAN_PREFILL = 8
 LF_TEST_WITHHOLD_PARTIALS = 0x100
 NOALLOC_SCRATCH_BYTES = 8 * 1024 * 1024
 ABI_VERSION = 4
+
+# Per device index, filled by the operators' Python paths: fit for the kernels
+# (gfx950), and compute units.
+ARCH_OK: dict = {}
+COMPUTE_UNITS: dict = {}
+# Cached workspaces: (device index, stream) for the fused calls, ("rows",
+# device index, stream) for the row shrink (ops/fused.py::_workspace).
+WORKSPACES: dict = {}
 
 _lock = threading.Lock()
 _handle: ctypes.CDLL | None = None
@@ -166,6 +175,53 @@ def library() -> ctypes.CDLL:
                 raise RuntimeError("loraforge_amd native library ABI mismatch; rebuild it")
             _handle = lib
     return _handle
+
+
+_binding_module = None
+
+
+def binding():
+    """The operators' native call path (``csrc/host/binding.cpp``), bound to the loaded library.
+
+    Its functions return None for any call they do not take; the operator's
+    Python code then serves or refuses it. ``ARCH_OK`` and ``COMPUTE_UNITS``
+    tell it which devices were found fit, ``WORKSPACES`` is the cache that it
+    finds the current stream's workspace in.
+    """
+    global _binding_module
+    if _binding_module is not None:
+        return _binding_module
+    import importlib.machinery
+    import importlib.util
+
+    import torch
+
+    lib = library()
+    with _lock:
+        if _binding_module is None:
+            if not BINDING.exists():
+                raise RuntimeError(f"loraforge_amd native binding missing at {BINDING}; build it with `python -m loraforge_amd._build`")
+            loader = importlib.machinery.ExtensionFileLoader("_binding", str(BINDING))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_binding", str(BINDING), loader=loader))
+            loader.exec_module(module)
+            entries = (
+                lib.lf_nf4_lora_linear,
+                lib.lf_nf4_lora_workspace_size,
+                lib.lf_lora_apply,
+                lib.lf_row_shrink,
+                lib.lf_row_shrink_workspace_size,
+                lib.lf_row_expand,
+                lib.lf_nf4_dequant,
+            )
+            stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+                lambda index: torch.cuda.current_stream(index).cuda_stream
+            )
+            device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+            module.init(
+                tuple(ctypes.cast(fn, ctypes.c_void_p).value for fn in entries), stream, device, ARCH_OK, WORKSPACES, COMPUTE_UNITS
+            )
+            _binding_module = module
+    return _binding_module
 
 
 def check(status: int) -> None:

@@ -11,6 +11,8 @@ from __future__ import annotations
 
 import functools
 
+from .. import _lib
+
 ARCH = "gfx950"
 
 
@@ -53,5 +55,7 @@ def require_arch(device) -> None:
     """The kernels are built for gfx950 only (the reference pins gfx90a, ops/nf4.py:68-75)."""
     import torch
 
-    if not torch.version.hip or _arch(device.index if device.index is not None else torch.cuda.current_device()) != ARCH:
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    if not torch.version.hip or _arch(index) != ARCH:
         raise RuntimeError(f"loraforge_amd kernels require ROCm {ARCH}")
+    _lib.ARCH_OK[index] = True

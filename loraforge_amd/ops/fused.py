@@ -27,7 +27,8 @@ from ..annotations import ExperimentalAPI
 from ._checks import distinct_output, require_arch, tensor, vector
 
 _WS_LOCK = threading.Lock()
-_WORKSPACES: dict = {}
+_WORKSPACES = _lib.WORKSPACES
+_PLAN_FLAGS = {None: 0, "decode": _lib.LF_PLAN_DECODE_CHUNKS, "prefill": _lib.LF_PLAN_PREFILL}
 _RETIRED: list = []  # replaced workspaces a captured graph may still address
 
 
@@ -318,6 +319,10 @@ def nf4_lora_linear(
 
     if plan not in (None, "prefill", "decode"):
         raise ValueError("plan must be None, 'prefill' or 'decode'")
+    if workspace is None and getattr(x, "is_cuda", False):
+        done = _lib.binding().linear(x, qweight, state, scales, bias, lora, out, exact, swiglu, _PLAN_FLAGS[plan])
+        if done is not None:
+            return done
     if not isinstance(x, torch.Tensor) or not isinstance(qweight, torch.Tensor):
         raise TypeError("x and qweight must be tensors")
     if state.quant_type != "nf4" or state.blocksize != 64:
@@ -403,7 +408,7 @@ def nf4_lora_linear(
                 workspace.numel(),
                 (_lib.LF_EXACT_WEIGHTS if exact else 0)
                 | (_lib.LF_SWIGLU_OUTPUT if swiglu else 0)
-                | {None: 0, "decode": _lib.LF_PLAN_DECODE_CHUNKS, "prefill": _lib.LF_PLAN_PREFILL}[plan],
+                | _PLAN_FLAGS[plan],
                 stream,
             )
         )
@@ -430,6 +435,10 @@ def lora_apply(x, y, lora: LoraBatch, *, workspace=None):
         raise TypeError("x and y must be tensors")
     if not isinstance(lora, LoraBatch):
         raise TypeError("lora must be a LoraBatch")
+    if workspace is None and getattr(x, "is_cuda", False):
+        done = _lib.binding().apply(x, y, lora)
+        if done is not None:
+            return done
     device = x.device
     if device.type != "cuda" or y.device != device:
         raise ValueError("all tensors must be on the same CUDA/ROCm GPU")

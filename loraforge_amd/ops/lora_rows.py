@@ -57,6 +57,8 @@ def row_shrink(
     """
     import torch
 
+    if getattr(x, "is_cuda", False) and _lib.binding().shrink(x, a, output, slots, ranks, num_slices, max_rank):
+        return
     tensor(x, "x", 2, torch.bfloat16)
     tensor(a, "a", 3, torch.bfloat16, x.device)
     tensor(output, "output", 2, torch.bfloat16, x.device)
@@ -146,6 +148,11 @@ def row_expand(
     """
     import torch
 
+    if getattr(z, "is_cuda", False) and _lib.binding().expand(
+        z, b, output, b_offsets, b_strides, ranks, scales, segment_indptr, segment_slots, token_indices, slice_offsets,
+        segment_count, blocks, threads,
+    ):
+        return
     tensor(z, "z", 2, torch.bfloat16)
     tensor(b, "b", 1, torch.bfloat16, z.device)
     tensor(output, "output", 2, torch.bfloat16, z.device)
@@ -197,7 +204,9 @@ def row_expand(
     lib = _lib.library()
     with torch.cuda.device(z.device):
         if blocks is None:
-            blocks = 2 * torch.cuda.get_device_properties(z.device).multi_processor_count
+            units = torch.cuda.get_device_properties(z.device).multi_processor_count
+            _lib.COMPUTE_UNITS[z.device.index] = units
+            blocks = 2 * units
         _lib.check(
             lib.lf_row_expand(
                 z.data_ptr(),

@@ -207,6 +207,10 @@ def dequantize_nf4(qweight, scales, code, shape: tuple[int, int], *, out=None):
     """
     import torch
 
+    if out is None and getattr(qweight, "is_cuda", False):
+        done = _lib.binding().dequant(qweight, scales, code, shape)
+        if done is not None:
+            return done
     if (
         not isinstance(shape, tuple)
         or len(shape) != 2

@@ -1,0 +1,115 @@
+"""The operators' native call path (``csrc/host/binding.cpp``) against their Python path.
+
+Every form the native path takes must give the Python path's bits, and every
+call it declines must be served, or refused with the same error, as before:
+the second call of a shape runs natively, a call with ``workspace=`` or with
+the native path switched off runs in Python.
+"""
+
+import pytest
+import torch
+
+from loraforge_amd import _lib
+from loraforge_amd.ops import dequantize_nf4, lora_apply, nf4_lora_linear, row_expand, row_shrink
+from tests import _cases
+from tests.test_fused_gpu import to_device
+
+pytestmark = pytest.mark.gpu
+
+
+class _Declines:
+    """Stands in for the binding: every call goes the Python way."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def both(monkeypatch, call):
+    call()  # warms the device flags and the workspace
+    taken = call()
+    with monkeypatch.context() as patch:
+        patch.setattr(_lib, "_binding_module", _Declines())
+        python = call()
+    torch.cuda.synchronize()
+    return taken, python
+
+
+@pytest.mark.parametrize("dq", [False, True])
+@pytest.mark.parametrize("m,lead,swiglu,bias", [(1, None, False, True), (6, (2, 3), False, False), (9, None, True, False),
+                                                (80, None, True, False), (96, (3, 32), False, True)])
+def test_linear_forms(m, lead, swiglu, bias, dq, device, monkeypatch):
+    bounds = [0, 256, 512] if swiglu else None
+    case = _cases.fused_case(m, 512, 320, ranks=(16, 8, 4), slices=2 if swiglu else 1, bounds=bounds, double_quant=dq,
+                             bias=bias, seed=400 + m)
+    x, q, st, lora, b = to_device(case, device)
+    x = x if lead is None else x.reshape(*lead, -1)
+    wide = torch.zeros(m, x.shape[-1] + 64, dtype=torch.bfloat16, device=device)
+    forms = [dict(lora=lora), dict(lora=None), dict(lora=lora, exact=True), dict(lora=lora, plan="decode")]
+    if dq:
+        forms.append(dict(lora=lora, scales="nested"))
+    for kw in forms:
+        taken, python = both(monkeypatch, lambda: nf4_lora_linear(x, q, st, bias=b, swiglu=swiglu, **kw))
+        assert taken.shape == python.shape and torch.equal(taken, python), kw
+    if lead is None:
+        strided = wide[:, : x.shape[-1]].copy_(x)
+        taken, python = both(monkeypatch, lambda: nf4_lora_linear(strided, q, st, bias=b, swiglu=swiglu, lora=lora))
+        assert torch.equal(taken, python)
+        out = torch.empty(m, 520, dtype=torch.bfloat16, device=device)[:, : 256 if swiglu else 512]
+        taken, python = both(monkeypatch, lambda: nf4_lora_linear(x, q, st, bias=b, swiglu=swiglu, lora=lora, out=out).clone())
+        assert torch.equal(taken, python)
+
+
+def test_prepared_scales_follow_an_update(device, monkeypatch):
+    """A nested state whose tensors change in place is prepared again, not served from the cached scales."""
+    case = _cases.fused_case(4, 256, 512, ranks=(8,), double_quant=True, seed=431)
+    x, q, st, lora, _ = to_device(case, device)
+    before, _ = both(monkeypatch, lambda: nf4_lora_linear(x, q, st, lora=lora))
+    st.state2.absmax.mul_(2.0)
+    after, python = both(monkeypatch, lambda: nf4_lora_linear(x, q, st, lora=lora))
+    assert torch.equal(after, python) and not torch.equal(after, before)
+
+
+def test_row_operators_and_dequant(device, monkeypatch):
+    c = _cases.c2_case(seed=441, tokens=24, k=512, n=256, adapters=4)
+    t = lambda a: torch.from_numpy(a.view("int16") if a.dtype == "uint16" else a).to(device)
+    bf = lambda a: t(a).view(torch.bfloat16)
+    x, a, b = bf(c["x"]), bf(c["a"]), bf(c["b"])
+    routes = t(c["routes"])
+    meta = {k: t(v) for k, v in c["meta"].items()}
+
+    def rows():
+        z, y = bf(c["z"]).clone(), bf(c["y"]).clone()
+        row_shrink(x, a, z, routes, meta["ranks"], max_rank=16)
+        row_expand(z, b, y, **meta)
+        return torch.cat([z.reshape(-1), y.reshape(-1)])
+
+    taken, python = both(monkeypatch, rows)
+    assert torch.equal(taken, python)
+    case = _cases.fused_case(24, 256, 512, ranks=(16, 8), seed=442)
+    xl, q, st, lora, _ = to_device(case, device)
+    base = torch.randn(24, 256, device=device).bfloat16()
+    taken, python = both(monkeypatch, lambda: lora_apply(xl, base.clone(), lora))
+    assert torch.equal(taken, python)
+    taken, python = both(monkeypatch, lambda: dequantize_nf4(q, st.absmax, st.code, (256, 512)))
+    assert torch.equal(taken, python)
+
+
+def test_refusals_are_the_python_path_s(device):
+    """What the operators refuse they refuse after native calls too, with their own messages."""
+    case = _cases.fused_case(4, 256, 512, ranks=(8, 4), seed=451)
+    x, q, st, lora, _ = to_device(case, device)
+    for _ in range(2):
+        good = nf4_lora_linear(x, q, st, lora=lora)
+    with pytest.raises(ValueError, match="inference-only"):
+        nf4_lora_linear(x.clone().requires_grad_(), q, st, lora=lora)
+    with pytest.raises(ValueError, match="unit column stride"):
+        nf4_lora_linear(x[:, ::2], q, st, lora=lora)
+    with pytest.raises(ValueError, match="share storage"):
+        nf4_lora_linear(x, q, st, out=x[:, :256])
+    with pytest.raises(ValueError, match="token_slots"):
+        nf4_lora_linear(x, q, st, lora=lora.with_tokens(lora.token_slots[:2]))
+    with pytest.raises(ValueError, match="nested"):
+        nf4_lora_linear(x, q, st, scales="nested")
+    with pytest.raises(ValueError, match="16-entry"):
+        dequantize_nf4(q, st.absmax, st.code[:8], (256, 512))
+    assert torch.equal(nf4_lora_linear(x, q, st, lora=lora), good)
