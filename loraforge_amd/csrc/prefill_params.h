@@ -52,8 +52,10 @@ struct PrefillParams {
 // tile heights, so that they compile side by side).
 template <int RI>
 int launch_rows(const PrefillParams& p, int64_t blocks, bool lora, bool swiglu, hipStream_t stream);
-// Launches the z producers alone (mtiles * zparts workgroups).
+// Launches the z producers alone (mtiles * zparts workgroups; zflags may be null).
 int launch_z(const PrefillParams& p, hipStream_t stream);
+// y += LoRA for p.m tokens from finished z rows (lora_apply_tiles.hip).
+int launch_apply_z(const PrefillParams& p, hipStream_t stream);
 
 }  // namespace prefill
 }  // namespace lf

@@ -392,12 +392,16 @@ __device__ __forceinline__ void store_z(uint16_t* dst, uint16_t v) {
 }
 
 constexpr int kUnit = 16;        // tokens per unit
-constexpr int kUnitRows = 64;    // A rows per pass
 
-// kUnitSteps: k steps of loads in flight per wave (8 in the producers' own
-// launch; 4 in the GEMM launch, whose registers hold no more beside the tile).
-template <int kUnitSteps>
-__device__ void produce_units(const PrefillParams& p, int mt, int q, int* tslot, int* list, int* order, int* cnt,
+// kUnitSteps: k steps of loads in flight per wave. kRowTiles: 16-row tiles of A
+// per pass; kRowParts: workgroups that share a unit's rows (this one takes the
+// passes rp, rp + kRowParts, ...). In the producers' own launch 16 steps of
+// one tile, four workgroups a unit: a fragment load (16 rows, 64 bytes of
+// each) takes the address unit 64 cycles, so a unit is bound by the loads of
+// one CU. In the GEMM launch 4 steps of four tiles (its registers hold no more
+// beside the output tile).
+template <int kUnitSteps, int kRowTiles, int kRowParts, int kThreads = prefill::kThreads>
+__device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int* tslot, int* list, int* order, int* cnt,
                               int* ustart, float* red) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -405,6 +409,7 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int* tslot,
   const int c = lane & 15;
   const int kg = lane >> 4;
   constexpr int kWaves = kThreads / 64;
+  constexpr int kPassRows = 16 * kRowTiles;
   const int m0 = mt * p.tile_rows;
   const int count = min(p.tile_rows, p.m - m0);
   const int zw = p.slices * kZSlice;
@@ -456,7 +461,7 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int* tslot,
   __syncthreads();
   // Zero the padding columns r .. 63 of every slice of the tokens this producer serves.
   const int units = ustart[nd];
-  for (int u = q; u < units; u += p.zparts) {
+  for (int u = rp == 0 ? q : units; u < units; u += p.zparts) {
     int d = 0;
     while (ustart[d + 1] <= u) ++d;
     const int first = cnt[d] + (u - ustart[d]) * kUnit;
@@ -479,20 +484,20 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int* tslot,
     const uint16_t* abase = p.a_store + p.a_offsets[gd];
     const int tok = m0 + order[first + min(c, ntok - 1)];
     const uint16_t* xrow = p.x + int64_t(tok) * p.x_stride + 8 * kg;
-    for (int j0 = 0; j0 < rows; j0 += kUnitRows) {
-      f32x4 acc[4];
+    for (int j0 = rp * kPassRows; j0 < rows; j0 += kRowParts * kPassRows) {
+      f32x4 acc[kRowTiles];
 #pragma unroll
-      for (int jt = 0; jt < 4; ++jt) acc[jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-      const int tiles = (min(kUnitRows, rows - j0) + 15) >> 4;  // uniform
+      for (int jt = 0; jt < kRowTiles; ++jt) acc[jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      const int tiles = (min(kPassRows, rows - j0) + 15) >> 4;  // uniform
       for (int s0 = wave; s0 < steps; s0 += kWaves * kUnitSteps) {
         // Loads of this batch's steps first (past the end: a readable step, not contracted).
-        uint4 xb[kUnitSteps], ab[kUnitSteps][4];
+        uint4 xb[kUnitSteps], ab[kUnitSteps][kRowTiles];
 #pragma unroll
         for (int v = 0; v < kUnitSteps; ++v) {
           const int st = min(s0 + v * kWaves, steps - 1);
           xb[v] = *reinterpret_cast<const uint4*>(xrow + st * 32);
 #pragma unroll
-          for (int jt = 0; jt < 4; ++jt)
+          for (int jt = 0; jt < kRowTiles; ++jt)
             if (jt < tiles)
               ab[v][jt] = *reinterpret_cast<const uint4*>(abase + int64_t(min(j0 + jt * 16 + c, rows - 1)) * p.k +
                                                           st * 32 + 8 * kg);
@@ -501,23 +506,23 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int* tslot,
         for (int v = 0; v < kUnitSteps; ++v)
           if (s0 + v * kWaves < steps)
 #pragma unroll
-            for (int jt = 0; jt < 4; ++jt)
+            for (int jt = 0; jt < kRowTiles; ++jt)
               if (jt < tiles) acc[jt] = mfma16(as_bf16x8(ab[v][jt]), as_bf16x8(xb[v]), acc[jt]);
       }
       // acc[jt][e] = this wave's partial of z[token c][A row j0 + 16 jt + 4 kg + e].
 #pragma unroll
-      for (int jt = 0; jt < 4; ++jt)
+      for (int jt = 0; jt < kRowTiles; ++jt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) red[((wave * 4 + jt) * 16 + 4 * kg + e) * 17 + c] = acc[jt][e];
+        for (int e = 0; e < 4; ++e) red[((wave * kRowTiles + jt) * 16 + 4 * kg + e) * 17 + c] = acc[jt][e];
       __syncthreads();
-      for (int o = tid; o < kUnitRows * kUnit; o += kThreads) {
+      for (int o = tid; o < kPassRows * kUnit; o += kThreads) {
         const int jr = o >> 4;  // A row within the pass
         const int t = o & 15;
         const int j = j0 + jr;
         if (t < ntok && j < rows) {
           float sum = 0.f;
 #pragma unroll
-          for (int w = 0; w < kWaves; ++w) sum += red[((w * 4 + (jr >> 4)) * 16 + (jr & 15)) * 17 + t];
+          for (int w = 0; w < kWaves; ++w) sum += red[((w * kRowTiles + (jr >> 4)) * 16 + (jr & 15)) * 17 + t];
           const int sl = j / r;
           store_z(p.zpad + int64_t(m0 + order[first + t]) * zw + sl * kZSlice + (j - sl * r), uint16_t(f32_to_bf16(sum)));
         }
@@ -533,12 +538,12 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int* tslot,
 }
 
 // Producer (mt, q): its units, then its flag carries the call's tag.
-template <int kUnitSteps>
-__device__ __forceinline__ void produce_z(const PrefillParams& p, int mt, int q, uint32_t tag, int* tslot, int* list,
+template <int kUnitSteps, int kRowTiles, int kRowParts, int kThreads = prefill::kThreads>
+__device__ __forceinline__ void produce_z(const PrefillParams& p, int mt, int q, int rp, uint32_t tag, int* tslot, int* list,
                                           int* order, int* cnt, int* ustart, float* red) {
   if (p.withhold) return;  // test hook: the tile's consumers must recompute
-  produce_units<kUnitSteps>(p, mt, q, tslot, list, order, cnt, ustart, red);
-  if (threadIdx.x == 0) __hip_atomic_store(p.zflags + mt * p.zparts + q, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  produce_units<kUnitSteps, kRowTiles, kRowParts, kThreads>(p, mt, q, rp, tslot, list, order, cnt, ustart, red);
+  if (threadIdx.x == 0 && p.zflags) __hip_atomic_store(p.zflags + mt * p.zparts + q, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Waits until the z rows of M-tile mt carry the call's tag (their producers
@@ -570,7 +575,7 @@ __device__ bool wait_z(const PrefillParams& p, int mt, uint32_t tag, int* tslot,
   if (lost == 0) return false;
   if (threadIdx.x == 0) __hip_atomic_store(p.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (int q = 0; q < p.zparts; ++q)
-    if ((lost >> q) & 1) produce_units<4>(p, mt, q, tslot, list, order, mrank, mstride, red);
+    if ((lost >> q) & 1) produce_units<4, 4, 1>(p, mt, q, 0, tslot, list, order, mrank, mstride, red);
   int tid = threadIdx.x;
   tie(tid);  // (opaque: nothing of this rare path is kept from before the k-loop)
   for (int d = tid; d < list[kMaxList]; d += kThreads) {
@@ -645,12 +650,16 @@ __device__ __forceinline__ int tile_row(const PrefillParams& p, int nt, int r) {
 // The producers as a launch of their own, ahead of the GEMM's on the same
 // stream. It takes the call's tag but leaves counting in (and so moving the
 // epoch on) to the GEMM launch, which finds every flag set.
-__global__ __launch_bounds__(kThreads) void z_kernel(PrefillParams p) {
-  __shared__ __attribute__((aligned(16))) float red[kMinRing / 4];
+// (Eight waves, so that a wave's share of K = 4096 is one batch of loads.)
+constexpr int kZThreads = 512;
+constexpr int kZRowParts = 4;
+__global__ __launch_bounds__(kZThreads) void z_kernel(PrefillParams p) {
+  __shared__ __attribute__((aligned(16))) float red[kZThreads / 64 * 16 * 17];
   __shared__ __attribute__((aligned(16))) int tslot[kBM];
   __shared__ int list[kMaxList + 1], order[kBM], cnt[kMaxList + 1], ustart[kMaxList + 1];
-  const uint32_t tag = __builtin_amdgcn_readfirstlane(epoch_tag(p.ce));
-  produce_z<8>(p, blockIdx.x / p.zparts, blockIdx.x % p.zparts, tag, tslot, list, order, cnt, ustart, red);
+  const uint32_t tag = p.zflags ? __builtin_amdgcn_readfirstlane(epoch_tag(p.ce)) : 0u;
+  const int unit = blockIdx.x / kZRowParts;
+  produce_z<16, 1, kZRowParts, kZThreads>(p, unit / p.zparts, unit % p.zparts, blockIdx.x % kZRowParts, tag, tslot, list, order, cnt, ustart, red);
 }
 
 // Block ids below zblocks (LoRA launches whose last round has room for them)
@@ -692,7 +701,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(PrefillParams pk) {
     if (b < p.zblocks) {
       // (The slot metadata arrays double as the producer's sort counters; the
       // idle x ring holds the partial tiles.)
-      produce_z<4>(p, b / p.zparts, b % p.zparts, tag, tslot, list, order, mrank, mstride, reinterpret_cast<float*>(xring));
+      produce_z<4, 4, 1>(p, b / p.zparts, b % p.zparts, 0, tag, tslot, list, order, mrank, mstride, reinterpret_cast<float*>(xring));
       depart(p, tag);
       return;
     }
@@ -1166,7 +1175,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(PrefillParams pk) {
 
 #ifdef LF_PREFILL_Z_KERNEL
 int launch_z(const PrefillParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL(tile::z_kernel, dim3(p.mtiles * p.zparts), dim3(kThreads), 0, stream, p);
+  hipLaunchKernelGGL(tile::z_kernel, dim3(p.mtiles * p.zparts * tile::kZRowParts), dim3(tile::kZThreads), 0, stream, p);
   LF_HIP(hipGetLastError());
   return kOk;
 }
