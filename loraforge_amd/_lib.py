@@ -85,6 +85,10 @@ _PROTOTYPES = {
         ctypes.c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p],
     ),
+    "lf_nf4_dequant_dq_checked": (
+        ctypes.c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, ctypes.POINTER(c_int32), c_void_p],
+    ),
     "lf_nf4_prepare_scales_dq": (
         ctypes.c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p],
@@ -212,6 +216,7 @@ def binding():
                 lib.lf_row_shrink_workspace_size,
                 lib.lf_row_expand,
                 lib.lf_nf4_dequant,
+                lib.lf_nf4_dequant_dq_checked,
             )
             stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
                 lambda index: torch.cuda.current_stream(index).cuda_stream

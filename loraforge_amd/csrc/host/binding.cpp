@@ -32,6 +32,7 @@ decltype(&lf_row_shrink) g_shrink;
 decltype(&lf_row_shrink_workspace_size) g_shrink_ws;
 decltype(&lf_row_expand) g_expand;
 decltype(&lf_nf4_dequant) g_dequant;
+decltype(&lf_nf4_dequant_dq_checked) g_dequant_dq;
 
 PyObject* g_raw_stream;   // torch._C._cuda_getCurrentRawStream
 PyObject* g_get_device;   // torch._C._cuda_getDevice
@@ -534,18 +535,62 @@ PyObject* dequant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return THPVariable_Wrap(out);
 }
 
+// dequant_nested(qweight, state) -> out or None. The library checks the codebook
+// in the kernel: two blocking copies and a comparison launch per call before
+// (115 us at 24576 x 4096, the kernel itself 40).
+PyObject* dequant_nested(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 2) return decline();
+  PyObject* state = args[1];
+  const at::Tensor* q = plain(args[0]);
+  if (!q) return decline();
+  const at::Device dev = q->device();
+  Ref nested(PyObject_GetAttr(state, s_nested)), shape(PyObject_GetAttr(state, s_shape));
+  Ref absmax(PyObject_GetAttr(state, s_absmax)), code_o(PyObject_GetAttr(state, s_code));
+  if (!nested || !shape || !absmax || !code_o || nested.p != Py_True) return decline();
+  long n, k;
+  if (!PyTuple_Check(shape.p) || PyTuple_GET_SIZE(shape.p) != 2 ||
+      !small_int(PyTuple_GET_ITEM(shape.p, 0), 64, 1 << 28, &n) || !small_int(PyTuple_GET_ITEM(shape.p, 1), 64, 1 << 28, &k) ||
+      n % 64 || k % 64)
+    return decline();
+  const int64_t size = int64_t(n) * k;
+  const at::Tensor* code = plain(code_o.p);
+  if (q->scalar_type() != at::kByte || q->numel() != size / 2 || !q->is_contiguous() || !code || code->device() != dev ||
+      code->scalar_type() != at::kFloat || code->numel() != 16 || !code->is_contiguous())
+    return decline();
+  lf_nf4_weight w{};
+  NestedArg two;
+  if (!two.take(state, absmax.p, size / 64, dev, &w)) return decline();
+  void* stream;
+  if (!current(dev, &stream)) return decline();
+  at::Tensor out = at::empty({n, k}, code->options().dtype(at::kBFloat16));
+  if (!on_gpu(out)) return decline();
+  int rc = LF_OK;
+  int32_t canonical = 0;
+  uint16_t* dst = static_cast<uint16_t*>(out.data_ptr());
+  Py_BEGIN_ALLOW_THREADS
+  rc = g_dequant_dq(ptr<uint8_t>(q), w.absmax_q, w.absmax2, w.code2, w.offset, w.dq_block, ptr<float>(code), dst, size,
+                    &canonical, stream);
+  Py_END_ALLOW_THREADS
+  if (rc == LF_EINVAL || (rc == LF_OK && !canonical)) return decline();
+  if (rc != LF_OK) {
+    PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in dequantize_nf4_nested");
+    return nullptr;
+  }
+  return THPVariable_Wrap(out);
+}
+
 // init(addresses, raw_stream, get_device, arch_ok, workspaces, compute_units)
 PyObject* init(PyObject*, PyObject* args) {
   PyObject *addresses, *raw, *dev, *arch, *ws, *cus;
   if (!PyArg_ParseTuple(args, "O!OOO!O!O!", &PyTuple_Type, &addresses, &raw, &dev, &PyDict_Type, &arch, &PyDict_Type, &ws,
                         &PyDict_Type, &cus))
     return nullptr;
-  void* a[7];
-  if (PyTuple_GET_SIZE(addresses) != 7) {
-    PyErr_SetString(PyExc_ValueError, "seven entry points expected");
+  void* a[8];
+  if (PyTuple_GET_SIZE(addresses) != 8) {
+    PyErr_SetString(PyExc_ValueError, "eight entry points expected");
     return nullptr;
   }
-  for (int i = 0; i < 7; ++i)
+  for (int i = 0; i < 8; ++i)
     if (!(a[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(addresses, i)))) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null entry point");
       return nullptr;
@@ -557,6 +602,7 @@ PyObject* init(PyObject*, PyObject* args) {
   g_shrink_ws = reinterpret_cast<decltype(g_shrink_ws)>(a[4]);
   g_expand = reinterpret_cast<decltype(g_expand)>(a[5]);
   g_dequant = reinterpret_cast<decltype(g_dequant)>(a[6]);
+  g_dequant_dq = reinterpret_cast<decltype(g_dequant_dq)>(a[7]);
 #define INTERN(n) \
   if (!s_##n && !(s_##n = PyUnicode_InternFromString(#n))) return nullptr;
   NAMES(INTERN)
@@ -585,6 +631,7 @@ PyMethodDef methods[] = {
     {"apply", reinterpret_cast<PyCFunction>(guarded<apply>), METH_FASTCALL, nullptr},
     {"shrink", reinterpret_cast<PyCFunction>(guarded<shrink>), METH_FASTCALL, nullptr},
     {"expand", reinterpret_cast<PyCFunction>(guarded<expand>), METH_FASTCALL, nullptr},
+    {"dequant_nested", reinterpret_cast<PyCFunction>(guarded<dequant_nested>), METH_FASTCALL, nullptr},
     {"dequant", reinterpret_cast<PyCFunction>(guarded<dequant>), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -5,12 +5,21 @@
 // HBM-bound: per 64-element block it reads 32 packed bytes + 4 scale bytes
 // and writes 128 bytes. Each lane decodes one packed dword (8 elements) per
 // step and stores 16 bytes, so every load (256 B/wave) and store (1 KiB/wave)
-// instruction is fully coalesced. Two independent steps per lane (2048
-// workgroups at 8192 x 1024) measured best: 6.3 us against 7.1 us with four
-// and 7.2 us with one. Packed bytes at an address that is not 4-byte
+// instruction is fully coalesced. The stores are non-temporal: the output is
+// four times the packed bytes and larger than the caches can hold back, and
+// writing it through them cost half the rate (24576 x 4096: fp32 scales 55.7
+// -> 37.3 us, 257 MB at 6.9 TB/s; nested 72.5 -> 39.6 us; 8192 x 1024 5.6 ->
+// 4.3 us). Two independent steps per lane (one: 38.4 us, four: 37.7 us at
+// 24576 x 4096); four for a nested state of at least 32 M elements (39.6 us
+// against 44.7 us: fewer workgroups stage the 256-entry code2), two below
+// (4096 x 4096 7.5 us against 7.7 us). Packed bytes at an address that is not 4-byte
 // aligned, or an output that is not 16-byte aligned (a contiguous view at an
 // odd offset, which the reference accepts), take the same kernel with byte
 // loads and 2-byte stores.
+#include <atomic>
+#include <chrono>
+#include <mutex>
+
 #include "nf4_common.h"
 #include "../../include/loraforge_amd.h"
 
@@ -18,7 +27,7 @@ namespace lf {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kSteps = 2;
+constexpr int64_t kLargeNested = int64_t(32) << 20;  // elements: four steps per lane
 
 // Packed dword w of the weight (bytes 4w..4w+3, little endian).
 template <bool kAligned>
@@ -35,7 +44,7 @@ __device__ __forceinline__ uint32_t load_packed(const uint8_t* __restrict__ pack
 template <bool kAligned>
 __device__ __forceinline__ void store_elements(uint16_t* __restrict__ out, int64_t w, uint4 v) {
   if constexpr (kAligned) {
-    reinterpret_cast<uint4*>(out)[w] = v;
+    __builtin_nontemporal_store((u32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(out) + w);
   } else {
     uint16_t* p = out + 8 * w;
     const uint32_t words[4] = {v.x, v.y, v.z, v.w};
@@ -47,10 +56,38 @@ __device__ __forceinline__ void store_elements(uint16_t* __restrict__ out, int64
   }
 }
 
-template <bool kDouble, bool kAligned>
+// The canonical codebook (reference ops/nf4.py:120-141), which a checked call holds `code` to.
+__constant__ const float kCanonical[16] = {
+    -1.0f,
+    -0.6961928009986877f,
+    -0.5250730514526367f,
+    -0.39491748809814453f,
+    -0.28444138169288635f,
+    -0.18477343022823334f,
+    -0.09105003625154495f,
+    0.0f,
+    0.07958029955625534f,
+    0.16093020117282867f,
+    0.24611230194568634f,
+    0.33791524171829224f,
+    0.44070982933044434f,
+    0.5626170039176941f,
+    0.7229568362236023f,
+    1.0f,
+};
+
+// A checked call's answer: its ticket, and whether the codebook is canonical,
+// in one word of host memory (verdict null: unchecked).
+struct Verdict {
+  uint64_t* word;
+  uint32_t ticket;
+};
+
+template <bool kDouble, bool kAligned, int kSteps>
 __global__ __launch_bounds__(kThreads) void nf4_dequant_kernel(const uint8_t* __restrict__ packed,
                                                                ScaleSource src, const float* __restrict__ code,
-                                                               uint16_t* __restrict__ out, int64_t ndwords) {
+                                                               uint16_t* __restrict__ out, int64_t ndwords,
+                                                               Verdict verdict) {
   __shared__ float table[16];
   __shared__ float code2[kDouble ? 256 : 1];
   // Packed bytes are requested first; the codebook is staged while they travel.
@@ -65,6 +102,12 @@ __global__ __launch_bounds__(kThreads) void nf4_dequant_kernel(const uint8_t* __
   if (threadIdx.x < 16) table[threadIdx.x] = code[threadIdx.x];
   if constexpr (kDouble) code2[threadIdx.x] = src.code2[threadIdx.x];
   __syncthreads();
+  if (kDouble && verdict.word && blockIdx.x == 0 && threadIdx.x < 64) {
+    const uint64_t same = __ballot(threadIdx.x >= 16 || table[threadIdx.x & 15] == kCanonical[threadIdx.x & 15]);
+    if (threadIdx.x == 0)
+      __hip_atomic_store(verdict.word, (uint64_t(verdict.ticket) << 1) | (same == ~uint64_t(0) ? 1u : 0u), __ATOMIC_RELEASE,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 #pragma unroll
   for (int s = 0; s < kSteps; ++s) {
     const int64_t w = base + s * kThreads;
@@ -89,29 +132,84 @@ __global__ __launch_bounds__(kThreads) void dq_scales_kernel(ScaleSource src, fl
 }
 
 int launch_dequant(const uint8_t* qweight, const ScaleSource& src, const float* code, uint16_t* out,
-                   int64_t numel, void* stream) {
+                   int64_t numel, void* stream, Verdict verdict = Verdict{nullptr, 0}) {
   LF_REQUIRE(numel > 0 && numel % (kNf4Block * kNf4Block) == 0,
              "element count must be a positive multiple of 4096");
   LF_REQUIRE(qweight && code && out, "null pointer argument");
   LF_REQUIRE((reinterpret_cast<uintptr_t>(out) & 1u) == 0, "out must be 2-byte aligned (bf16)");
   const int64_t ndwords = numel / 8;
-  const int64_t grid = (ndwords + kThreads * kSteps - 1) / (kThreads * kSteps);
+  const int steps = !src.scales && numel >= kLargeNested ? 4 : 2;
+  const int64_t grid = (ndwords + kThreads * steps - 1) / (kThreads * steps);
   LF_REQUIRE(grid < (int64_t(1) << 31), "tensor too large");
   auto s = static_cast<hipStream_t>(stream);
   const bool vec = aligned16(out) && (reinterpret_cast<uintptr_t>(qweight) & 3u) == 0;
   if (src.scales) {
-    auto k = vec ? nf4_dequant_kernel<false, true> : nf4_dequant_kernel<false, false>;
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, s, qweight, src, code, out, ndwords);
+    auto k = vec ? nf4_dequant_kernel<false, true, 2> : nf4_dequant_kernel<false, false, 2>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, s, qweight, src, code, out, ndwords, verdict);
   } else {
-    auto k = vec ? nf4_dequant_kernel<true, true> : nf4_dequant_kernel<true, false>;
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, s, qweight, src, code, out, ndwords);
+    auto k = steps == 4 ? (vec ? nf4_dequant_kernel<true, true, 4> : nf4_dequant_kernel<true, false, 4>)
+                        : (vec ? nf4_dequant_kernel<true, true, 2> : nf4_dequant_kernel<true, false, 2>);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, s, qweight, src, code, out, ndwords, verdict);
   }
   LF_HIP(hipGetLastError());
   return kOk;
 }
 
+// Words for the answers of checked calls in flight (one per call, in turn).
+// Pinned host memory of one page, kept until the process ends.
+constexpr uint32_t kVerdicts = 256;
+std::mutex g_verdict_lock;
+uint64_t* g_verdicts = nullptr;
+std::atomic<uint32_t> g_ticket{0};
+
 }  // namespace
 }  // namespace lf
+
+extern "C" int lf_nf4_dequant_dq_checked(const uint8_t* qweight, const uint8_t* absmax_q, const float* absmax2,
+                                         const float* code2, const float* offset, int64_t dq_block, const float* code,
+                                         uint16_t* out, int64_t numel, int32_t* canonical, void* stream) {
+  LF_REQUIRE(absmax_q && absmax2 && code2 && offset && canonical, "double-quant state pointers required");
+  LF_REQUIRE(dq_block > 0 && dq_block <= (int64_t(1) << 30), "dq_block must be positive");
+  auto s = static_cast<hipStream_t>(stream);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  LF_HIP(hipStreamIsCapturing(s, &capture));
+  LF_REQUIRE(capture == hipStreamCaptureStatusNone, "a checked call waits for its answer: not under graph capture");
+  {
+    std::lock_guard<std::mutex> guard(lf::g_verdict_lock);
+    if (lf::g_verdicts == nullptr) {
+      void* page = nullptr;
+      LF_HIP(hipHostMalloc(&page, lf::kVerdicts * sizeof(uint64_t), hipHostMallocPortable));
+      for (uint32_t i = 0; i < lf::kVerdicts; ++i) static_cast<uint64_t*>(page)[i] = 0;
+      lf::g_verdicts = static_cast<uint64_t*>(page);
+    }
+  }
+  // (Ticket 0 is what an unused word holds.)
+  uint32_t ticket;
+  do ticket = lf::g_ticket.fetch_add(1, std::memory_order_relaxed) + 1;
+  while (ticket == 0);
+  uint64_t* word = lf::g_verdicts + ticket % lf::kVerdicts;
+  void* device_word = nullptr;
+  LF_HIP(hipHostGetDevicePointer(&device_word, word, 0));
+  lf::ScaleSource src{nullptr, absmax_q, absmax2, code2, offset, int(dq_block)};
+  const int rc = lf::launch_dequant(qweight, src, code, out, numel, stream,
+                                    lf::Verdict{static_cast<uint64_t*>(device_word), ticket});
+  if (rc != lf::kOk) return rc;
+  // The answer comes as the kernel starts: a short look for it, then the
+  // stream's own wait (work ahead of the kernel, or an error).
+  auto answered = [&](uint64_t* v) {
+    *v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    return uint32_t(*v >> 1) == ticket;
+  };
+  uint64_t v = 0;
+  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
+  while (!answered(&v)) {
+    if (std::chrono::steady_clock::now() < until) continue;
+    LF_HIP(hipStreamSynchronize(s));
+    if (!answered(&v)) return lf::fail(lf::kHip, "the codebook check gave no answer");
+  }
+  *canonical = int32_t(v & 1);
+  return lf::kOk;
+}
 
 extern "C" int lf_nf4_dequant(const uint8_t* qweight, const float* scales, const float* code, uint16_t* out,
                               int64_t numel, void* stream) {

@@ -264,6 +264,10 @@ def dequantize_nf4_nested(qweight, state, *, out=None):
 
     if not state.nested:
         return dequantize_nf4(qweight, state.absmax, state.code, tuple(state.shape), out=out)
+    if out is None and getattr(qweight, "is_cuda", False):
+        done = _lib.binding().dequant_nested(qweight, state)
+        if done is not None:
+            return done
     n, k = (int(v) for v in state.shape)
     device = qweight.device
     _checks.require_arch(device)

@@ -6,11 +6,21 @@ the second call of a shape runs natively, a call with ``workspace=`` or with
 the native path switched off runs in Python.
 """
 
+import dataclasses
+
 import pytest
 import torch
 
 from loraforge_amd import _lib
-from loraforge_amd.ops import dequantize_nf4, lora_apply, nf4_lora_linear, row_expand, row_shrink
+from loraforge_amd.ops import (
+    dequantize_nf4,
+    dequantize_nf4_nested,
+    lora_apply,
+    nf4_lora_linear,
+    quantize_nf4,
+    row_expand,
+    row_shrink,
+)
 from tests import _cases
 from tests.test_fused_gpu import to_device
 
@@ -92,6 +102,22 @@ def test_row_operators_and_dequant(device, monkeypatch):
     assert torch.equal(taken, python)
     taken, python = both(monkeypatch, lambda: dequantize_nf4(q, st.absmax, st.code, (256, 512)))
     assert torch.equal(taken, python)
+
+
+@pytest.mark.parametrize("n,k", [(64, 64), (192, 320), (4096, 8192)])
+def test_nested_dequant_checks_the_codebook(n, k, device, monkeypatch):
+    """Below and at the four-step size (32 M elements): bits of the Python path; a codebook with one other
+    value is refused, and so is the next call with it."""
+    g = torch.Generator(device=device).manual_seed(n + k)
+    q, st = quantize_nf4((torch.randn(n, k, generator=g, device=device) * 0.02).bfloat16(), compress_statistics=True)
+    taken, python = both(monkeypatch, lambda: dequantize_nf4_nested(q, st))
+    assert torch.equal(taken, python)
+    wrong = dataclasses.replace(st, code=st.code.clone())
+    wrong.code[11] += 1e-6
+    for _ in range(2):
+        with pytest.raises(ValueError, match="canonical"):
+            dequantize_nf4_nested(q, wrong)
+    assert torch.equal(dequantize_nf4_nested(q, st), python)
 
 
 def test_refusals_are_the_python_path_s(device):
