@@ -28,11 +28,12 @@
 //    pass z x B_g^T over the 32-token blocks holding its tokens gives the
 //    delta, applied with the reference's two bf16 roundings.
 //
-// What bounds it (4096 x 4096 x 12288, 96 stages, RI = 8, one round): MFMA
+// What bounds it (4096 x 4096 x 12288, 96 stages, RI = 8, one round; counters of a
+// 344 us form): MFMA
 // busy 66 % of 595 k cycles, the rest decode and copy issue; at that load the
 // part runs at about 1.8 GHz, so the energy of decode (-20 % time without it)
 // and of the x copies (-21 % without them) counts as much as their cycles.
-// 344 us against 481 us with the weights decoded cooperatively into LDS (tile
+// Now 323 us, against 480 us with the weights decoded cooperatively into LDS (tile
 // 256 x 192, LDS-bound); a library bf16 GEMM on dequantised weights takes 313 us.
 // Measured and rejected: the waves' copies in turns (uniform branches per
 // slot, 364 us), copies earlier in the stage (357-389 us).
@@ -825,17 +826,18 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(PrefillParams pk) {
       // enough for its shadow: decode pieces, a quarter of the next block's
       // codes (steps 2..5), copies of stage + 2's weights (step 0), of x of
       // stages + kR - 1 (four steps) and + kR (step 7), and in even stages the
-      // loads of the next pair's scales (step 6).
+      // loads of the next pair's scales (step 0: a use that the compiler had to
+      // wait for would also wait for the x copies behind them).
       auto step = [&](auto tc, XFrags<RI>& xc, u32x4 (&wc)[kJ], XFrags<RI>& xn, u32x4 (&wn)[kJ]) {
         constexpr int t = decltype(tc)::value;
         constexpr bool kLast = t == kSteps - 1;
         constexpr int kNext = (t + 1) % kSteps;
         if constexpr (kLast) {
-          // The next stage's x and the weights after it have landed once only
-          // the scale loads of step 6 (and, with three stages, this stage's x
-          // copies, all behind its weight copies) are outstanding; past the
-          // barrier this stage's x is free.
-          wait_vm<(kOdd ? 0 : kJ) + (kR > 2 ? 2 * RI - kFirstCopies<RI> : 0)>();
+          // The next stage's x, the weights after it and the next scales have
+          // landed once only this stage's x copies (three stages: all behind
+          // its weight copies and scale loads) or nothing (two stages) is
+          // outstanding; past the barrier this stage's x is free.
+          wait_vm<(kR > 2 ? 2 * RI - kFirstCopies<RI> : 0)>();
           barrier_only();
           read_x<RI>(there, xn);
           read_w(wl, cur);
@@ -877,7 +879,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(PrefillParams pk) {
                 if (m == f * kSlots / kJ + k * (kSlots / kJ) / 3)
                   build[f].phase(k, code, cs.s[f][kOdd ? 0 : 1], t - 2, ncodes[f]);
             }
-            if (!kOdd && t == 6 && m == (2 * f + 1) * kSlots / (2 * kJ)) load_scales(wl, w2, h, f, ns);
+            if (!kOdd && t == 0 && m == f) load_scales(wl, w2, h, f, ns);
           }
           if (t == 0) {
 #pragma unroll
@@ -903,10 +905,15 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(PrefillParams pk) {
       step(std::integral_constant<int, 6>{}, xa, wa, xb, wb);
       step(std::integral_constant<int, 7>{}, xb, wb, xa, wa);
     };
-    for (int st = 0; st < stages; st += 2) {
+    // (An odd last stage stands alone: a way around the odd stage inside the
+    // loop would make the compiler wait, at the top of every pair, for the
+    // scale loads that only the odd stage consumes, and with them for the x
+    // copies just issued.)
+    for (int st = 0; st + 1 < stages; st += 2) {
       stage(st, std::false_type{}, even, odd);
-      if (st + 1 < stages) stage(st + 1, std::true_type{}, odd, even);
+      stage(st + 1, std::true_type{}, odd, even);
     }
+    if (stages & 1) stage(last, std::false_type{}, even, odd);
     wait_vm<0>();  // the requests past the end
     barrier_only();
   }
