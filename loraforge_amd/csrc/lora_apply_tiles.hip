@@ -156,6 +156,7 @@ int launch_lora_apply_tiles(const uint16_t* x, int64_t m, int64_t x_stride, int6
   p.tile_rows = kBM;
   p.mtiles = int((m + kBM - 1) / kBM);
   p.zparts = 2 * kBM / 16;
+  p.zrow_parts = z_row_parts(p.slices, lora->max_rank);
   const int rc = launch_z(p, s);
   if (rc != kOk) return rc;
   p.tile_rows = kTokens;

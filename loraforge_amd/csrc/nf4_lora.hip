@@ -34,14 +34,14 @@ int launch_decode_wide(const uint16_t* x, int64_t m, int64_t x_stride, const lf_
                        bool exact, bool swiglu, bool withhold, void* stream);
 constexpr int64_t kDecodeMaxTokens = 64;
 
-double prefill_us(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu);
+double prefill_us(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu);
 
 // Whether the wide decode kernel (32 rows x 32 tokens per workgroup over the
 // whole K) serves M > 64 tokens faster than the prefill GEMM (prefill_us):
 // a round of 256 wide workgroups takes 7.5 us per 4096 of K, 8.8 us with LoRA
 // (its per-CU x and weight reads; 256 tokens x 4096: 30 / 40 us against 56 /
 // 65 us on the prefill GEMM, 256 x 11008: 98 us against 67 us).
-bool wide_cheaper(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) {
+bool wide_cheaper(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu) {
   const int64_t cus = device_cus();
   const int64_t wide_groups = ((n / 32 + 7) / 8) * 8 * ((m + 31) / 32);
   const double wide_us = double((wide_groups + cus - 1) / cus) * (lora ? 8.8 : 7.5) * double(k) / 4096.0;
@@ -54,7 +54,7 @@ bool wide_cheaper(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) {
 // uses every CU). A decode launch of 64 tokens streams its weight bytes
 // (packed + fp32 scales) at about 0.8 TB/s, plus about 6 us with LoRA (4096 x
 // 4096: 11.9 us base only, 18.0 us with 32 rank-16 adapters).
-bool decode_chunks_cheaper(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) {
+bool decode_chunks_cheaper(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu) {
   const double weight_bytes = double(n) * double(k) * (0.5 + 4.0 / 64.0);
   const double chunk_us = (lora ? 6.0 : 0.0) + weight_bytes / 0.8e6;
   const int64_t chunks = (m + kDecodeMaxTokens - 1) / kDecodeMaxTokens;
@@ -120,7 +120,7 @@ extern "C" int lf_nf4_lora_linear(const uint16_t* x, int64_t m, int64_t x_stride
   // unless the prefill GEMM is forced or cheaper, or the shape is outside the
   // kernel's range.
   if (lf::decode_wide_fits(m, n, k, lora) && !(flags & LF_PLAN_PREFILL) &&
-      (m <= lf::kDecodeMaxTokens || (flags & LF_PLAN_DECODE_CHUNKS) || lf::wide_cheaper(m, n, k, lora != nullptr, swiglu)))
+      (m <= lf::kDecodeMaxTokens || (flags & LF_PLAN_DECODE_CHUNKS) || lf::wide_cheaper(m, n, k, lora, swiglu)))
     return lf::launch_decode_wide(x, m, x_stride, w, bias, lora, y, y_stride, workspace, workspace_bytes, exact,
                                   swiglu, withhold, stream);
   if (m <= lf::kDecodeMaxTokens)
@@ -128,7 +128,7 @@ extern "C" int lf_nf4_lora_linear(const uint16_t* x, int64_t m, int64_t x_stride
                              withhold, stream);
   bool chunked = false;
   if (flags & LF_PLAN_DECODE_CHUNKS) chunked = true;
-  else if (!(flags & LF_PLAN_PREFILL)) chunked = lf::decode_chunks_cheaper(m, n, k, lora != nullptr, swiglu);
+  else if (!(flags & LF_PLAN_PREFILL)) chunked = lf::decode_chunks_cheaper(m, n, k, lora, swiglu);
   if (!chunked)
     return lf::launch_nf4_lora_prefill(x, m, x_stride, w, bias, lora, y, y_stride, workspace, workspace_bytes,
                                        swiglu, withhold, stream);

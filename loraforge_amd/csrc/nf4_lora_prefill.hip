@@ -37,16 +37,20 @@ int zparts_in_slack(int64_t mtiles, int64_t tiles, int64_t cus) {
 }
 
 // Tile heights that are built, in 32-token fragments, and the time of a round
-// of such tiles at K = 4096 (us, a full chip, no LoRA; measured at 2048 x 11008
-// x 4096 and 4096 x 4096 x 12288). Below 4 fragments the decode of the tile's
-// weights (the same for every height) bounds it instead of the MFMAs.
+// of such tiles per 4096 of K (us; between a full chip, which runs at a lower
+// clock, and a few tiles). Below 4 fragments the decode of the tile's weights
+// (the same for every height) bounds it instead of the MFMAs.
 struct TileCost {
   int ri;
   double us;
 };
-constexpr TileCost kTileCosts[] = {{8, 108.0}, {6, 88.0}, {5, 75.0}, {4, 69.0}, {3, 61.0}, {2, 46.0}};
-constexpr double kZLaunchUs = 14.0;  // a round of z producers of one unit each at K = 4096
-constexpr double kLoraRoundUs = 10.0;  // a tile's z and B reads and its expand
+constexpr TileCost kTileCosts[] = {{8, 100.0}, {6, 82.0}, {5, 72.0}, {4, 64.0}, {3, 58.0}, {2, 52.0}};
+// What a round takes beside its k-loop: start, rounding and stores, and with
+// LoRA routes, z and B reads and the expand (1024 x 4096 x 1024, rank 16, heights
+// 8 .. 3: 47 / 37 / 35 / 32 / 29 us, of which the k-loop is 25 .. 14).
+double round_us(int ri, bool lora) { return lora ? 9.0 + 1.2 * ri : 4.0 + 0.6 * ri; }
+// A round of z producers of one unit each, one workgroup per CU.
+double z_round_us(int64_t k) { return 12.0 + 6.0 * double(k) / 4096.0; }
 
 struct TilePlan {
   int ri;
@@ -57,10 +61,12 @@ struct TilePlan {
 };
 
 // The tile height whose rounds of one tile per CU take the least time: 2048 x
-// 11008 (43 column tiles) runs in two rounds of 192-token tiles (190 us)
-// instead of two of 256 (204 us), 300 tokens x 24576 (SwiGLU) in one round of
-// 160-token tiles (77 us against 98 us).
-TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) {
+// 11008 x 4096 (43 column tiles) runs in two rounds of 192-token tiles (186 us)
+// instead of two of 256 (208 us), 300 tokens x 24576 (SwiGLU) in one round of
+// 160-token tiles (77 us against 98 us), 4096 x 4096 x 1024 with LoRA in two
+// of 160 tokens (64 us) instead of one of 256, whose z would be a launch of
+// its own.
+TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int slices, int max_rank, bool lora, bool swiglu) {
   const int64_t cus = device_cus();
   const int64_t ntiles = ((swiglu ? n / 2 : n) + (swiglu ? kTileN / 2 : kTileN) - 1) / (swiglu ? kTileN / 2 : kTileN);
   TilePlan best{};
@@ -69,14 +75,15 @@ TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) {
     p.mtiles = (m + 32 * c.ri - 1) / (32 * c.ri);
     if (p.mtiles > kMaxFlags) continue;
     p.tiles = p.mtiles * ntiles;
-    p.us = double((p.tiles + cus - 1) / cus) * (c.us * double(k) / 4096.0 + (lora ? kLoraRoundUs : 0.0));
+    p.us = double((p.tiles + cus - 1) / cus) * (c.us * double(k) / 4096.0 + round_us(c.ri, lora));
     if (lora) {
       p.zparts = zparts_in_slack(p.mtiles, p.tiles, cus);
       p.z_launch = p.zparts == 0;
       if (p.z_launch) {
-        // A producer per 16 tokens; two of its workgroups fit a CU.
-        p.zparts = int(std::max<int64_t>(1, std::min<int64_t>(2 * c.ri, kMaxFlags / p.mtiles)));
-        p.us += kZLaunchUs * double(k) / 4096.0 * double((p.mtiles * p.zparts + 2 * cus - 1) / (2 * cus));
+        // A producer per 16 tokens, and two for the units that slot changes add.
+        p.zparts = int(std::max<int64_t>(1, std::min<int64_t>(2 * c.ri + 2, kMaxFlags / p.mtiles)));
+        const int64_t groups = p.mtiles * p.zparts * z_row_parts(slices, max_rank);
+        p.us += z_round_us(k) * double((groups + cus - 1) / cus);
       }
     }
     if (best.ri == 0 || p.us < best.us) best = p;
@@ -84,7 +91,9 @@ TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) {
   return best;
 }
 
-double prefill_us(int64_t m, int64_t n, int64_t k, bool lora, bool swiglu) { return tile_plan(m, n, k, lora, swiglu).us; }
+double prefill_us(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu) {
+  return tile_plan(m, n, k, lora ? lora->num_slices : 1, lora ? lora->max_rank : 1, lora != nullptr, swiglu).us;
+}
 
 int64_t prefill_workspace_bytes(int64_t m, int64_t n, int64_t k, int slices, int) {
   return kWorkspaceHeader + kFlagRegion + align256(m * slices * kZSlice * 2) + align256(n * (k / kNf4Block) * 4);
@@ -153,10 +162,11 @@ int launch_nf4_lora_prefill(const uint16_t* x, int64_t m, int64_t x_stride, cons
   // SwiGLU output: each tile takes kBN / 2 activation columns (their gate and
   // up rows) and stores 16-byte chunks of them.
   LF_REQUIRE(!swiglu || p.y_vec == 2, "prefill SwiGLU output needs y 16-byte aligned with row stride %% 8 == 0");
-  const TilePlan plan = tile_plan(m, w->n, w->k, lora != nullptr, swiglu);
+  const TilePlan plan = tile_plan(m, w->n, w->k, slices, lora ? lora->max_rank : 1, lora != nullptr, swiglu);
   p.tile_rows = 32 * plan.ri;
   p.mtiles = int(plan.mtiles);
   p.zparts = plan.zparts;
+  p.zrow_parts = z_row_parts(slices, lora ? lora->max_rank : 1);
   // LoRA launches put the z producers ahead of the GEMM tiles.
   p.zblocks = lora && !plan.z_launch ? p.mtiles * p.zparts : 0;
   const int64_t blocks = plan.tiles + p.zblocks;

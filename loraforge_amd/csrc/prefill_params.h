@@ -42,6 +42,7 @@ struct PrefillParams {
   int* status;  // set to 1 if a wait for z gives up (cannot happen while producers run first)
   int mtiles;
   int zparts;   // z producers per M-tile
+  int zrow_parts;  // workgroups of the producers' own launch that share a unit's A rows
   int zblocks;  // producers among this launch's workgroups (0: none, or a launch of their own)
   int tile_rows;  // tokens per M-tile
   int spin_limit;  // polls of the bounded wait for a producer's flag
@@ -52,7 +53,12 @@ struct PrefillParams {
 // tile heights, so that they compile side by side).
 template <int RI>
 int launch_rows(const PrefillParams& p, int64_t blocks, bool lora, bool swiglu, hipStream_t stream);
-// Launches the z producers alone (mtiles * zparts workgroups; zflags may be null).
+// 16-row passes over a unit's A rows, at most four: workgroups that share them.
+inline int z_row_parts(int slices, int max_rank) {
+  const int passes = (slices * max_rank + 15) / 16;
+  return passes < 4 ? passes : 4;
+}
+// Launches the z producers alone (mtiles * zparts * zrow_parts workgroups; zflags may be null).
 int launch_z(const PrefillParams& p, hipStream_t stream);
 // y += LoRA for p.m tokens from finished z rows (lora_apply_tiles.hip).
 int launch_apply_z(const PrefillParams& p, hipStream_t stream);

@@ -28,15 +28,16 @@
 //    pass z x B_g^T over the 32-token blocks holding its tokens gives the
 //    delta, applied with the reference's two bf16 roundings.
 //
-// What bounds it (4096 x 4096 x 12288, 96 stages, RI = 8, one round; counters of a
-// 344 us form): MFMA
-// busy 66 % of 595 k cycles, the rest decode and copy issue; at that load the
-// part runs at about 1.8 GHz, so the energy of decode (-20 % time without it)
-// and of the x copies (-21 % without them) counts as much as their cycles.
-// Now 323 us, against 480 us with the weights decoded cooperatively into LDS (tile
-// 256 x 192, LDS-bound); a library bf16 GEMM on dequantised weights takes 313 us.
-// Measured and rejected: the waves' copies in turns (uniform branches per
-// slot, 364 us), copies earlier in the stage (357-389 us).
+// What bounds it (4096 x 4096 x 12288, 96 stages, RI = 8, one round; counters of
+// a 344 us form): MFMA busy 66 % of 595 k cycles, the rest decode and copy
+// issue; at that load the part runs at about 1.8 GHz, so the energy of the
+// decode (-20 % time without it) and of the x copies (-21 % without them)
+// counts as much as their cycles. Now 323 us, against 480 us with the weights
+// decoded cooperatively into LDS (tile 256 x 192, LDS-bound); a library bf16
+// GEMM on dequantised weights takes 313 us. Measured and rejected: the waves'
+// copies in turns (uniform branches per slot, 364 us), copies earlier in the
+// stage (357-389 us), K split over two groups of waves in a 64-token tile (two
+// waves per SIMD: 51.6 us against 53.6 us at 128 x 24576 x 4096, slower with LoRA).
 #pragma once
 
 #include <type_traits>
@@ -395,14 +396,14 @@ __device__ __forceinline__ void store_z(uint16_t* dst, uint16_t v) {
 constexpr int kUnit = 16;        // tokens per unit
 
 // kUnitSteps: k steps of loads in flight per wave. kRowTiles: 16-row tiles of A
-// per pass; kRowParts: workgroups that share a unit's rows (this one takes the
-// passes rp, rp + kRowParts, ...). In the producers' own launch 16 steps of
-// one tile, four workgroups a unit: a fragment load (16 rows, 64 bytes of
+// per pass; parts: workgroups that share a unit's rows (this one takes the
+// passes rp, rp + parts, ...). In the producers' own launch 16 steps of
+// one tile, up to four workgroups a unit: a fragment load (16 rows, 64 bytes of
 // each) takes the address unit 64 cycles, so a unit is bound by the loads of
 // one CU. In the GEMM launch 4 steps of four tiles (its registers hold no more
 // beside the output tile).
-template <int kUnitSteps, int kRowTiles, int kRowParts, int kThreads = prefill::kThreads>
-__device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int* tslot, int* list, int* order, int* cnt,
+template <int kUnitSteps, int kRowTiles, int kThreads = prefill::kThreads>
+__device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int parts, int* tslot, int* list, int* order, int* cnt,
                               int* ustart, float* red) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -485,7 +486,7 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
     const uint16_t* abase = p.a_store + p.a_offsets[gd];
     const int tok = m0 + order[first + min(c, ntok - 1)];
     const uint16_t* xrow = p.x + int64_t(tok) * p.x_stride + 8 * kg;
-    for (int j0 = rp * kPassRows; j0 < rows; j0 += kRowParts * kPassRows) {
+    for (int j0 = rp * kPassRows; j0 < rows; j0 += parts * kPassRows) {
       f32x4 acc[kRowTiles];
 #pragma unroll
       for (int jt = 0; jt < kRowTiles; ++jt) acc[jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -539,11 +540,11 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
 }
 
 // Producer (mt, q): its units, then its flag carries the call's tag.
-template <int kUnitSteps, int kRowTiles, int kRowParts, int kThreads = prefill::kThreads>
-__device__ __forceinline__ void produce_z(const PrefillParams& p, int mt, int q, int rp, uint32_t tag, int* tslot, int* list,
+template <int kUnitSteps, int kRowTiles, int kThreads = prefill::kThreads>
+__device__ __forceinline__ void produce_z(const PrefillParams& p, int mt, int q, int rp, int parts, uint32_t tag, int* tslot, int* list,
                                           int* order, int* cnt, int* ustart, float* red) {
   if (p.withhold) return;  // test hook: the tile's consumers must recompute
-  produce_units<kUnitSteps, kRowTiles, kRowParts, kThreads>(p, mt, q, rp, tslot, list, order, cnt, ustart, red);
+  produce_units<kUnitSteps, kRowTiles, kThreads>(p, mt, q, rp, parts, tslot, list, order, cnt, ustart, red);
   if (threadIdx.x == 0 && p.zflags) __hip_atomic_store(p.zflags + mt * p.zparts + q, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -576,7 +577,7 @@ __device__ bool wait_z(const PrefillParams& p, int mt, uint32_t tag, int* tslot,
   if (lost == 0) return false;
   if (threadIdx.x == 0) __hip_atomic_store(p.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (int q = 0; q < p.zparts; ++q)
-    if ((lost >> q) & 1) produce_units<4, 4, 1>(p, mt, q, 0, tslot, list, order, mrank, mstride, red);
+    if ((lost >> q) & 1) produce_units<4, 4>(p, mt, q, 0, 1, tslot, list, order, mrank, mstride, red);
   int tid = threadIdx.x;
   tie(tid);  // (opaque: nothing of this rare path is kept from before the k-loop)
   for (int d = tid; d < list[kMaxList]; d += kThreads) {
@@ -653,14 +654,13 @@ __device__ __forceinline__ int tile_row(const PrefillParams& p, int nt, int r) {
 // epoch on) to the GEMM launch, which finds every flag set.
 // (Eight waves, so that a wave's share of K = 4096 is one batch of loads.)
 constexpr int kZThreads = 512;
-constexpr int kZRowParts = 4;
 __global__ __launch_bounds__(kZThreads) void z_kernel(PrefillParams p) {
   __shared__ __attribute__((aligned(16))) float red[kZThreads / 64 * 16 * 17];
   __shared__ __attribute__((aligned(16))) int tslot[kBM];
   __shared__ int list[kMaxList + 1], order[kBM], cnt[kMaxList + 1], ustart[kMaxList + 1];
   const uint32_t tag = p.zflags ? __builtin_amdgcn_readfirstlane(epoch_tag(p.ce)) : 0u;
-  const int unit = blockIdx.x / kZRowParts;
-  produce_z<16, 1, kZRowParts, kZThreads>(p, unit / p.zparts, unit % p.zparts, blockIdx.x % kZRowParts, tag, tslot, list, order, cnt, ustart, red);
+  const int unit = blockIdx.x / p.zrow_parts;
+  produce_z<16, 1, kZThreads>(p, unit / p.zparts, unit % p.zparts, blockIdx.x % p.zrow_parts, p.zrow_parts, tag, tslot, list, order, cnt, ustart, red);
 }
 
 // Block ids below zblocks (LoRA launches whose last round has room for them)
@@ -702,7 +702,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(PrefillParams pk) {
     if (b < p.zblocks) {
       // (The slot metadata arrays double as the producer's sort counters; the
       // idle x ring holds the partial tiles.)
-      produce_z<4, 4, 1>(p, b / p.zparts, b % p.zparts, 0, tag, tslot, list, order, mrank, mstride, reinterpret_cast<float*>(xring));
+      produce_z<4, 4>(p, b / p.zparts, b % p.zparts, 0, 1, tag, tslot, list, order, mrank, mstride, reinterpret_cast<float*>(xring));
       depart(p, tag);
       return;
     }
@@ -1182,7 +1182,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(PrefillParams pk) {
 
 #ifdef LF_PREFILL_Z_KERNEL
 int launch_z(const PrefillParams& p, hipStream_t stream) {
-  hipLaunchKernelGGL(tile::z_kernel, dim3(p.mtiles * p.zparts * tile::kZRowParts), dim3(tile::kZThreads), 0, stream, p);
+  hipLaunchKernelGGL(tile::z_kernel, dim3(p.mtiles * p.zparts * p.zrow_parts), dim3(tile::kZThreads), 0, stream, p);
   LF_HIP(hipGetLastError());
   return kOk;
 }
