@@ -60,6 +60,21 @@ bool decode_chunks_cheaper(int64_t m, int64_t n, int64_t k, const lf_lora* lora,
   const int64_t chunks = (m + kDecodeMaxTokens - 1) / kDecodeMaxTokens;
   return double(chunks) * chunk_us < prefill_us(m, n, k, lora, swiglu);
 }
+// Whether lora_apply's two launches over all tokens are cheaper than a launch
+// of the decode kernel's residual form per 64 tokens. Their time grows with
+// the distinct adapters of a tile (500 tokens x 5120 x 4096, 4 adapters: 31 us
+// against 142 us; 382 x 4096 x 1024, 8 adapters: 50 / 53 us; 300 x 1024 x 1024
+// over 32: 110 / 42 us; 300 x 4096 x 4096 over 128: 210 / 82 us), a launch per 64
+// tokens takes 8 us and 8 us more per 4096 x 4096; above 16 adapters (or a
+// pool of unknown size) the latter.
+bool apply_tiles_cheaper(int64_t m, int64_t n, int64_t k, int num_slots) {
+  if (num_slots < 1 || num_slots > 16) return false;
+  const double size = double(n) * double(k) / (4096.0 * 4096.0);
+  const double tiles_us = (14.0 + 4.2 * num_slots) * std::max(1.0, size);
+  const double launches_us = double((m + kDecodeMaxTokens - 1) / kDecodeMaxTokens) * (8.0 + 8.0 * size);
+  return tiles_us < launches_us;
+}
+
 // One decode launch of up to 64 tokens: the wide kernel for the batches and
 // shapes it takes (above 8 tokens, above 2 at N >= 8192, above 16 at
 // K > 8192), else the narrow one (the kernel a direct call of these rows
@@ -192,11 +207,11 @@ extern "C" int lf_lora_apply(const uint16_t* x, int64_t m, int64_t x_stride, int
   shape.n = n;
   shape.k = k;
   const bool withhold = (flags & LF_TEST_WITHHOLD_PARTIALS) != 0;
-  // Above 64 tokens: shrink and expand as two launches over all tokens whose z
-  // rows the workspace holds (500 tokens x 5120 x 4096, three slices: 31 us
-  // against eight 64-token launches of 17.6 us). A workspace that holds
+  // Above 64 tokens, where it is cheaper: shrink and expand as two launches
+  // over all tokens whose z rows the workspace holds. A workspace that holds
   // fewer than 128 tokens' rows takes the launches per 64 tokens below.
-  const int64_t fit = m > lf::kDecodeMaxTokens && !withhold && workspace && lf::aligned16(workspace)
+  const int64_t fit = m > lf::kDecodeMaxTokens && !withhold && workspace && lf::aligned16(workspace) &&
+                              lf::apply_tiles_cheaper(m, n, k, lora->num_slots)
                           ? lf::apply_tiles_tokens(workspace_bytes, lora->num_slices)
                           : 0;
   if (fit >= 128) {

@@ -20,10 +20,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize(
     "m,n,k,slices,bounds,ranks",
     [
-        (65, 64, 64, 1, None, (16, 1, 33)),  # one token past the 64-token launch; the smallest N and K
-        (96, 320, 192, 3, [0, 190, 257, 320], (64, 7, 0, 16)),  # slice bounds inside fragments, a wave past N
-        (257, 576, 320, 2, [0, 300, 576], (2, 4, 8, 17, 48)),  # a second 256-token z tile of one token
-        (300, 1024, 1024, 1, None, tuple([4, 8, 16, 32] * 16)),  # 64 slots: more z units than producers
+        (193, 64, 64, 1, None, (16,)),  # the fewest tokens that take the two launches; the smallest N and K
+        (257, 320, 192, 3, [0, 190, 257, 320], (64, 7, 0, 16)),  # slice bounds inside fragments, a wave past N; a second z tile of one token
+        (330, 576, 320, 2, [0, 300, 576], (2, 4, 8, 17, 48)),  # a last tile of ten tokens
+        (700, 1024, 1024, 1, None, tuple([4, 8, 16, 32] * 4)),  # 16 slots: the most that take the two launches
+        (300, 1024, 256, 1, None, tuple([4, 8, 16, 32] * 16)),  # 64 slots: launches per 64 tokens
     ],
 )
 def test_tiles(m, n, k, slices, bounds, ranks, device):
