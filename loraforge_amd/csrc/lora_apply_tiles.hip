@@ -119,9 +119,14 @@ int launch_apply_z(const PrefillParams& p, hipStream_t stream) {
 
 }  // namespace prefill
 
-// Tokens whose z rows the workspace holds behind its control header.
+// z rows lie behind the control header and the flag region: a flag word of the
+// prefill GEMM may only ever hold tags, and z bits left there by a call on a
+// shared workspace could equal the tag of a later one.
+constexpr int64_t kZOffset = kWorkspaceHeader + kFlagRegion;
+
+// Tokens whose z rows the workspace holds.
 int64_t apply_tiles_tokens(int64_t workspace_bytes, int slices) {
-  return (workspace_bytes - kWorkspaceHeader) / (slices * prefill::kZSlice * 2);
+  return (workspace_bytes - kZOffset) / (slices * prefill::kZSlice * 2);
 }
 
 // y += LoRA(x) for m tokens (at most apply_tiles_tokens), two launches.
@@ -150,7 +155,7 @@ int launch_lora_apply_tiles(const uint16_t* x, int64_t m, int64_t x_stride, int6
   p.slice_offsets = lora->slice_offsets;
   p.slices = lora->num_slices;
   p.num_slots = lora->num_slots;
-  p.zpad = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + kWorkspaceHeader);
+  p.zpad = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + kZOffset);
   // z: a producer per 16-token unit of a 256-token tile, twice as many as one
   // slot would need (tokens of many slots make smaller units).
   p.tile_rows = kBM;

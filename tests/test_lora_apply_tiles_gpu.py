@@ -50,10 +50,11 @@ def test_routes_in_segments_and_a_workspace_of_few_tokens(device):
     x, y, batch = on_device(case, device)
     lora_apply(x, y, batch)
     check(case, y)
-    header = 262144
+    flags, header = 262144, 262144 + 16384  # the prefill flags' region ahead of the z rows stays untouched
     for rows, same in ((300, True), (100, False)):
         ws = torch.zeros(max(header + rows * 128, workspace_bytes(64, n, k, max_rank=32)), dtype=torch.uint8, device=device)
         _, again, _ = on_device(case, device)
         lora_apply(x, again, batch, workspace=ws)
         check(case, again)
         assert not same or np.array_equal(bits(again), bits(y))
+        assert not ws[flags:header].any()
