@@ -418,7 +418,8 @@ def nf4_lora_linear(
 
 @ExperimentalAPI(reason="gfx950 one-launch row_shrink + row_expand; caller-owned device metadata.")
 def lora_apply(x, y, lora: LoraBatch, *, workspace=None):
-    """``y += LoRA(x)`` in place for every routed token, one launch per 64 tokens.
+    """``y += LoRA(x)`` in place for every routed token: one launch per 64 tokens or, over
+    at most 16 adapters and where cheaper, two launches over all tokens.
 
     The reference chain ``row_shrink`` then ``row_expand``
     (``ops/lora_rows.py:51-239``) without materialising z or building
