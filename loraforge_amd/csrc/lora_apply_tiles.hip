@@ -10,8 +10,9 @@
 // read and written once. Bound by latency (z, B, then y) at a few hundred
 // tokens: 32-token tiles give 320 workgroups at 500 tokens x 5120.
 //
-// 500 tokens x 5120 x 4096, three slices of rank 16, four adapters: z 14.7 us and this
-// kernel 13.5 us, the call 142 -> 31 us (eight launches of the decode kernel before).
+// 500 tokens x 5120 x 4096, three slices of rank 16, four adapters: z 14.9 us and this
+// kernel 11.4 us (13.5 us with y read behind z B^T), the call 28.7 us (142 us as eight
+// launches of the decode kernel).
 #include <algorithm>
 
 #include "prefill_tile.h"
@@ -44,6 +45,16 @@ __global__ __launch_bounds__(kThreads) void apply_z_kernel(PrefillParams p) {
   for (int s = 0; s < 3; ++s)
     if (s < p.slices)
       zr[s] = *reinterpret_cast<const uint4*>(p.zpad + int64_t(zrow) * zw + s * kZSlice + (tid & 7) * 8);
+  const int wn0 = nt * kTileN + wave * 64;
+  uint16_t* yrow = p.y + int64_t(min(m0 + c, p.m - 1)) * p.y_stride + wn0;
+  // (Each value of y is updated by one slot and slice, so it can be read ahead of them all.
+  // N % 64 == 0: a wave's columns are all inside or all past N.)
+  uint2 yold[2][4];
+  if (p.y_vec && wn0 < p.n)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) yold[j][q] = *reinterpret_cast<const uint2*>(yrow + 32 * j + 8 * q + 4 * h);
   live_slots(p, m0, count, tslot, list);
   const int nd = list[kMaxList];
   if (nd == 0) return;
@@ -51,9 +62,7 @@ __global__ __launch_bounds__(kThreads) void apply_z_kernel(PrefillParams p) {
   for (int s = 0; s < 3; ++s)
     if (s < p.slices) zs[s][swz(tid >> 3, tid & 7)] = tslot[tid >> 3] >= 0 ? zr[s] : make_uint4(0, 0, 0, 0);
   __syncthreads();
-  const int wn0 = nt * kTileN + wave * 64;
-  if (wn0 >= p.n) return;  // N % 64 == 0: a wave's columns are all inside or all past N
-  uint16_t* yrow = p.y + int64_t(min(m0 + c, p.m - 1)) * p.y_stride + wn0;
+  if (wn0 >= p.n) return;
   for (int d = 0; d < nd; ++d) {
     const int gd = list[d];
     const int rank = p.ranks[gd];
@@ -92,7 +101,7 @@ __global__ __launch_bounds__(kThreads) void apply_z_kernel(PrefillParams p) {
           const uint32_t t23 = pack_bf16x2(delta[4 * q + 2] * scale, delta[4 * q + 3] * scale);
           uint16_t* dst = yrow + col;
           if (p.y_vec && n >= lo && n + 3 < hi) {
-            const uint2 old = *reinterpret_cast<const uint2*>(dst);
+            const uint2 old = yold[j][q];
             *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(bf16_lo(old.x) + bf16_lo(t01), bf16_hi(old.x) + bf16_hi(t01)),
                                                         pack_bf16x2(bf16_lo(old.y) + bf16_lo(t23), bf16_hi(old.y) + bf16_hi(t23)));
           } else {
