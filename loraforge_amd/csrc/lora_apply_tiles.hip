@@ -10,8 +10,8 @@
 // read and written once. Bound by latency (z, B, then y) at a few hundred
 // tokens: 32-token tiles give 320 workgroups at 500 tokens x 5120.
 //
-// 500 tokens x 5120 x 4096, three slices of rank 16, four adapters: z 14.9 us and this
-// kernel 11.4 us (13.5 us with y read behind z B^T), the call 28.7 us (142 us as eight
+// 500 tokens x 5120 x 4096, three slices of rank 16, four adapters: z 10.0 us and this
+// kernel 11.4 us (13.5 us with y read behind z B^T), the call 24.6 us (142 us as eight
 // launches of the decode kernel).
 #include <algorithm>
 

@@ -395,16 +395,85 @@ __device__ __forceinline__ void store_z(uint16_t* dst, uint16_t v) {
 
 constexpr int kUnit = 16;        // tokens per unit
 
-// kUnitSteps: k steps of loads in flight per wave. kRowTiles: 16-row tiles of A
-// per pass; parts: workgroups that share a unit's rows (this one takes the
-// passes rp, rp + parts, ...). In the producers' own launch 16 steps of
-// one tile, up to four workgroups a unit: a fragment load (16 rows, 64 bytes of
-// each) takes the address unit 64 cycles, so a unit is bound by the loads of
-// one CU. In the GEMM launch 4 steps of four tiles (its registers hold no more
+// One 16-row pass of a unit through LDS: a wave's 128-k stages wave, wave + kWaves,
+// ... of the unit's x rows and the A rows j0 .. j0 + 15 are copied as whole
+// 256-byte row pieces (four rows a copy) into the wave's own two slots of 8 KiB,
+// the next stage in flight behind the one contracted; waves do not meet.
+// Row r's 16-byte unit u sits at u ^ r. Past K the last unit is repeated (a
+// readable place, not contracted).
+// A unit is bound by one CU's loads: fragments straight from memory (16 rows, 64
+// bytes of each) take the address unit 64 cycles a load, a copy of whole 256-byte
+// pieces 16. The calls that launch it, fragment loads -> copies: lora_apply 500 x
+// 5120 x 4096 (three slices of rank 16) 28.7 -> 25.4 us, 1000 tokens of rank 64 80 ->
+// 53 us (more workgroups than CUs, at one per CU: still the faster form), 4096 x 4096 x
+// 4096 74 -> 66 us; the prefill linear 2048 x 8192 x 4096 of rank 64 170 -> 160 us.
+constexpr int kZSlot = 8192;
+template <int kWaves>
+__device__ __forceinline__ f32x4 contract_staged(const PrefillParams& p, const uint16_t* abase, int j0, int rows, int m0,
+                                                 const int* unit, int ntok, char* ring) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, kg = lane >> 4;
+  const int stages = (p.k + kBK - 1) / kBK;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  if (wave >= stages) return acc;
+  const char* xr[4];
+  const char* ar[4];
+  int at[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 4 * i + (lane >> 4);
+    xr[i] = reinterpret_cast<const char*>(p.x + int64_t(m0 + unit[min(r, ntok - 1)]) * p.x_stride);
+    ar[i] = reinterpret_cast<const char*>(abase + int64_t(min(j0 + r, rows - 1)) * p.k);
+    at[i] = ((lane & 15) ^ r) * 16;
+  }
+  char* mine = ring + wave * 2 * kZSlot;
+  auto issue = [&](int st, char* slot) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int off = min(st * (kBK * 2) + at[i], p.k * 2 - 16);
+      copy16(xr[i] + off, slot + i * 1024);
+      copy16(ar[i] + off, slot + kZSlot / 2 + i * 1024);
+    }
+  };
+  issue(wave, mine);
+  if (wave + kWaves < stages) issue(wave + kWaves, mine + kZSlot);
+  int n = 0;
+  for (int st = wave; st < stages; st += kWaves, n ^= 1) {
+    if (st + kWaves < stages) wait_vm<8>();  // all but the next stage's copies
+    else wait_vm<0>();
+    asm volatile("" ::: "memory");
+    const uint32_t base = lds_addr(mine) + uint32_t(n * kZSlot + c * 256);
+    u32x4 xv[4], av[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const uint32_t addr = base + uint32_t(((4 * v + kg) ^ c) << 4);
+      xv[v] = ldsr128<0>(addr);
+      av[v] = ldsr128<kZSlot / 2>(addr);
+    }
+    lds_wait();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      tie(xv[v]);
+      tie(av[v]);
+    }
+    if (st + 2 * kWaves < stages) issue(st + 2 * kWaves, mine + n * kZSlot);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (st * kBK + v * 32 < p.k) acc = mfma16(vec_bf16x8(av[v]), vec_bf16x8(xv[v]), acc);
+  }
+  return acc;
+}
+
+// kUnitSteps: k steps of loads in flight per wave, 0: through LDS
+// (contract_staged). kRowTiles: 16-row tiles of A per pass; parts: workgroups that
+// share a unit's rows (this one takes the passes rp, rp + parts, ...). In the
+// producers' own launch through LDS, one tile a pass, up to four workgroups a
+// unit. In the GEMM launch 4 steps of four tiles (its registers hold no more
 // beside the output tile).
 template <int kUnitSteps, int kRowTiles, int kThreads = prefill::kThreads>
 __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int parts, int* tslot, int* list, int* order, int* cnt,
-                              int* ustart, float* red) {
+                              int* ustart, float* red, char* ring = nullptr) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -491,7 +560,9 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
 #pragma unroll
       for (int jt = 0; jt < kRowTiles; ++jt) acc[jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
       const int tiles = (min(kPassRows, rows - j0) + 15) >> 4;  // uniform
-      for (int s0 = wave; s0 < steps; s0 += kWaves * kUnitSteps) {
+      if constexpr (kUnitSteps == 0) {
+        acc[0] = contract_staged<kWaves>(p, abase, j0, rows, m0, order + first, ntok, ring);
+      } else for (int s0 = wave; s0 < steps; s0 += kWaves * kUnitSteps) {
         // Loads of this batch's steps first (past the end: a readable step, not contracted).
         uint4 xb[kUnitSteps], ab[kUnitSteps][kRowTiles];
 #pragma unroll
@@ -542,9 +613,9 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
 // Producer (mt, q): its units, then its flag carries the call's tag.
 template <int kUnitSteps, int kRowTiles, int kThreads = prefill::kThreads>
 __device__ __forceinline__ void produce_z(const PrefillParams& p, int mt, int q, int rp, int parts, uint32_t tag, int* tslot, int* list,
-                                          int* order, int* cnt, int* ustart, float* red) {
+                                          int* order, int* cnt, int* ustart, float* red, char* ring = nullptr) {
   if (p.withhold) return;  // test hook: the tile's consumers must recompute
-  produce_units<kUnitSteps, kRowTiles, kThreads>(p, mt, q, rp, parts, tslot, list, order, cnt, ustart, red);
+  produce_units<kUnitSteps, kRowTiles, kThreads>(p, mt, q, rp, parts, tslot, list, order, cnt, ustart, red, ring);
   if (threadIdx.x == 0 && p.zflags) __hip_atomic_store(p.zflags + mt * p.zparts + q, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -652,15 +723,16 @@ __device__ __forceinline__ int tile_row(const PrefillParams& p, int nt, int r) {
 // The producers as a launch of their own, ahead of the GEMM's on the same
 // stream. It takes the call's tag but leaves counting in (and so moving the
 // epoch on) to the GEMM launch, which finds every flag set.
-// (Eight waves, so that a wave's share of K = 4096 is one batch of loads.)
+// (Eight waves: their 128 KiB of copies in flight fill the CU.)
 constexpr int kZThreads = 512;
 __global__ __launch_bounds__(kZThreads) void z_kernel(PrefillParams p) {
+  __shared__ __attribute__((aligned(256))) char ring[kZThreads / 64 * 2 * kZSlot];
   __shared__ __attribute__((aligned(16))) float red[kZThreads / 64 * 16 * 17];
   __shared__ __attribute__((aligned(16))) int tslot[kBM];
   __shared__ int list[kMaxList + 1], order[kBM], cnt[kMaxList + 1], ustart[kMaxList + 1];
   const uint32_t tag = p.zflags ? __builtin_amdgcn_readfirstlane(epoch_tag(p.ce)) : 0u;
   const int unit = blockIdx.x / p.zrow_parts;
-  produce_z<16, 1, kZThreads>(p, unit / p.zparts, unit % p.zparts, blockIdx.x % p.zrow_parts, p.zrow_parts, tag, tslot, list, order, cnt, ustart, red);
+  produce_z<0, 1, kZThreads>(p, unit / p.zparts, unit % p.zparts, blockIdx.x % p.zrow_parts, p.zrow_parts, tag, tslot, list, order, cnt, ustart, red, ring);
 }
 
 // Block ids below zblocks (LoRA launches whose last round has room for them)

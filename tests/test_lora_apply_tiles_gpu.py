@@ -58,3 +58,20 @@ def test_routes_in_segments_and_a_workspace_of_few_tokens(device):
         check(case, again)
         assert not same or np.array_equal(bits(again), bits(y))
         assert not ws[flags:header].any()
+
+
+@pytest.mark.parametrize(
+    "m,n,k,slices,bounds,ranks",
+    [
+        (200, 512, 2112, 1, None, (16, 3)),  # 16.5 stages of 128 k: one wave with three, the last of half a stage
+        (333, 256, 3136, 2, [0, 64, 256], (64, 5, 33)),  # 24.5 stages; units of several passes
+        (65, 1024, 4096, 1, None, (1,)),  # four stages a wave; one A row; a unit of one token
+    ],
+)
+def test_z_stages(m, n, k, slices, bounds, ranks, device):
+    """K where the waves of a z unit have different numbers of stages, and reuse their slots."""
+    routes = np.arange(m, dtype=np.int32) % (len(ranks) + 1) - 1 if len(ranks) > 1 else np.zeros(m, np.int32)
+    case = make_case(m, n, k, ranks, slices=slices, bounds=bounds, seed=m + k, routes=routes)
+    x, y, batch = on_device(case, device)
+    lora_apply(x, y, batch)
+    check(case, y)
