@@ -49,7 +49,10 @@ constexpr TileCost kTileCosts[] = {{8, 100.0}, {6, 82.0}, {5, 72.0}, {4, 64.0}, 
 // LoRA routes, z and B reads and the expand (1024 x 4096 x 1024, rank 16, heights
 // 8 .. 3: 47 / 37 / 35 / 32 / 29 us, of which the k-loop is 25 .. 14).
 double round_us(int ri, bool lora) { return lora ? 9.0 + 1.2 * ri : 4.0 + 0.6 * ri; }
-// A round of z producers of one unit each, one workgroup per CU.
+// A round of z producers of one unit each, one workgroup per CU, in a launch of
+// its own. (More than the kernel's own time, 9-10 us a round at K = 4096: at 5 + rounds x
+// (2.5 + 3 K / 4096) the rule takes the launch in sixteen of four hundred drawn shapes more,
+// and all of them get slower, 1292 x 13824 x 6144 245 -> 266 us.)
 double z_round_us(int64_t k) { return 12.0 + 6.0 * double(k) / 4096.0; }
 
 struct TilePlan {
