@@ -182,6 +182,28 @@ def library() -> ctypes.CDLL:
 
 
 _binding_module = None
+# The library's entry points that the native call path calls, in its order.
+_BOUND = (
+    "lf_nf4_lora_linear",
+    "lf_nf4_lora_workspace_size",
+    "lf_lora_apply",
+    "lf_row_shrink",
+    "lf_row_shrink_workspace_size",
+    "lf_row_expand",
+    "lf_nf4_dequant",
+    "lf_nf4_dequant_dq_checked",
+)
+
+
+def bind(module, **replaced) -> None:
+    """Hand the native call path its entry points (``replaced``: addresses that stand in for some)."""
+    import torch
+
+    stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda index: torch.cuda.current_stream(index).cuda_stream)
+    device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+    lib = library()
+    addresses = tuple(replaced.get(name) or ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _BOUND)
+    module.init(addresses, stream, device, ARCH_OK, WORKSPACES, COMPUTE_UNITS)
 
 
 def binding():
@@ -198,9 +220,9 @@ def binding():
     import importlib.machinery
     import importlib.util
 
-    import torch
+    import torch  # noqa: F401  (the module links to torch's libraries)
 
-    lib = library()
+    library()
     with _lock:
         if _binding_module is None:
             if not BINDING.exists():
@@ -208,23 +230,7 @@ def binding():
             loader = importlib.machinery.ExtensionFileLoader("_binding", str(BINDING))
             module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_binding", str(BINDING), loader=loader))
             loader.exec_module(module)
-            entries = (
-                lib.lf_nf4_lora_linear,
-                lib.lf_nf4_lora_workspace_size,
-                lib.lf_lora_apply,
-                lib.lf_row_shrink,
-                lib.lf_row_shrink_workspace_size,
-                lib.lf_row_expand,
-                lib.lf_nf4_dequant,
-                lib.lf_nf4_dequant_dq_checked,
-            )
-            stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
-                lambda index: torch.cuda.current_stream(index).cuda_stream
-            )
-            device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
-            module.init(
-                tuple(ctypes.cast(fn, ctypes.c_void_p).value for fn in entries), stream, device, ARCH_OK, WORKSPACES, COMPUTE_UNITS
-            )
+            bind(module)
             _binding_module = module
     return _binding_module
 

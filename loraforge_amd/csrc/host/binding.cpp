@@ -120,22 +120,36 @@ bool current(const at::Device& dev, void** stream) {
   return !PyErr_Occurred();
 }
 
-// The cached workspace of the current stream, if it holds `need` bytes.
-const at::Tensor* workspace(const at::Device& dev, void* stream, int64_t need, PyObject* kind) {
+// The cached workspace of the current stream, if it holds `need` bytes (else undefined).
+// (A reference of its own: the call is made without the GIL.)
+at::Tensor workspace(const at::Device& dev, void* stream, int64_t need, PyObject* kind) {
   Ref index(PyLong_FromLong(dev.index()));
   Ref s(PyLong_FromVoidPtr(stream));
   Ref key(kind ? PyTuple_Pack(3, kind, index.p, s.p) : PyTuple_Pack(2, index.p, s.p));
-  if (!key) return nullptr;
+  if (!key) return {};
   PyObject* ws = PyDict_GetItem(g_workspaces, key.p);
-  if (!ws || !THPVariable_CheckExact(ws)) return nullptr;
+  if (!ws || !THPVariable_CheckExact(ws)) return {};
   const at::Tensor& t = THPVariable_Unpack(ws);
-  return t.numel() >= need ? &t : nullptr;
+  return t.numel() >= need ? t : at::Tensor();
 }
 
 bool small_int(PyObject* o, long lo, long hi, long* out) {
   if (!o || !PyLong_CheckExact(o)) return false;
   *out = PyLong_AsLong(o);
   return !PyErr_Occurred() && *out >= lo && *out <= hi;
+}
+
+// A library call without the GIL: a launch blocks while the stream's queue is
+// full, which must not stop the process's other Python threads (one of them may
+// be what the queue waits for). What the call reads is referenced by the caller
+// or held above it.
+template <class F>
+int unlocked(F&& call) {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = call();
+  Py_END_ALLOW_THREADS
+  return rc;
 }
 
 template <class T>
@@ -339,8 +353,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!current(dev, &stream)) return decline();
   const int64_t need = g_linear_ws(m, n, k, has_lora ? lora.slices : 1, has_lora ? lora.d.max_rank : 1);
   if (need < 0) return decline();
-  const at::Tensor* ws = workspace(dev, stream, need, nullptr);
-  if (!ws) return decline();
+  const at::Tensor ws = workspace(dev, stream, need, nullptr);
+  if (!ws.defined()) return decline();
 
   at::Tensor result;
   int64_t y_stride = width;
@@ -365,9 +379,11 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   w.code = ptr<float>(code);
   w.n = n;
   w.k = k;
-  const int rc = g_linear(ptr<uint16_t>(x), m, x_stride, &w, ptr<uint16_t>(bias), has_lora ? &lora.d : nullptr,
-                          static_cast<uint16_t*>(result.data_ptr()), y_stride, ws->data_ptr(), ws->numel(),
-                          int32_t(flags) | (exact ? LF_EXACT_WEIGHTS : 0) | (swiglu ? LF_SWIGLU_OUTPUT : 0), stream);
+  const int rc = unlocked([&] {
+    return g_linear(ptr<uint16_t>(x), m, x_stride, &w, ptr<uint16_t>(bias), has_lora ? &lora.d : nullptr,
+                    static_cast<uint16_t*>(result.data_ptr()), y_stride, ws.data_ptr(), ws.numel(),
+                    int32_t(flags) | (exact ? LF_EXACT_WEIGHTS : 0) | (swiglu ? LF_SWIGLU_OUTPUT : 0), stream);
+  });
   if (rc == LF_EINVAL) return decline();  // (nothing was launched; the Python path raises the message)
   if (rc != LF_OK) {
     PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in nf4_lora_linear");
@@ -399,10 +415,12 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!current(dev, &stream)) return decline();
   const int64_t need = g_linear_ws(m < 64 ? m : 64, n, k, lora.slices, lora.d.max_rank);
   if (need < 0) return decline();
-  const at::Tensor* ws = workspace(dev, stream, need, nullptr);
-  if (!ws) return decline();
-  const int rc = g_apply(ptr<uint16_t>(x), m, x->stride(0), n, k, &lora.d, ptr<uint16_t>(y), y->stride(0), ws->data_ptr(),
-                         ws->numel(), 0, stream);
+  const at::Tensor ws = workspace(dev, stream, need, nullptr);
+  if (!ws.defined()) return decline();
+  const int rc = unlocked([&] {
+    return g_apply(ptr<uint16_t>(x), m, x->stride(0), n, k, &lora.d, ptr<uint16_t>(y), y->stride(0), ws.data_ptr(),
+                   ws.numel(), 0, stream);
+  });
   if (rc == LF_EINVAL) return decline();
   if (rc != LF_OK) {
     PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in lora_apply");
@@ -438,11 +456,13 @@ PyObject* shrink(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!current(dev, &stream)) return decline();
   const int64_t need = g_shrink_ws(m, width, g, int32_t(slices), int32_t(max_rank));
   if (need < 0) return decline();
-  const at::Tensor* ws = need ? workspace(dev, stream, need, s_rows) : nullptr;
-  if (need && !ws) return decline();
-  const int rc = g_shrink(ptr<uint16_t>(x), ptr<uint16_t>(a), ptr<uint16_t>(z), ptr<int32_t>(slots), ptr<int32_t>(ranks), m,
-                          width, x->stride(0), g, int32_t(slices), rows / slices, int32_t(max_rank),
-                          ws ? ws->data_ptr() : nullptr, ws ? ws->numel() : 0, 0, stream);
+  const at::Tensor ws = need ? workspace(dev, stream, need, s_rows) : at::Tensor();
+  if (need && !ws.defined()) return decline();
+  const int rc = unlocked([&] {
+    return g_shrink(ptr<uint16_t>(x), ptr<uint16_t>(a), ptr<uint16_t>(z), ptr<int32_t>(slots), ptr<int32_t>(ranks), m,
+                    width, x->stride(0), g, int32_t(slices), rows / slices, int32_t(max_rank),
+                    need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, 0, stream);
+  });
   if (rc == LF_EINVAL) return decline();
   if (rc != LF_OK) {
     PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in row_shrink");
@@ -492,10 +512,12 @@ PyObject* expand(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (shares(*y, {z, b, offsets, strides, ranks, scales, indptr, slots, tokens, bounds, count})) return decline();
   void* stream;
   if (!current(dev, &stream)) return decline();
-  const int rc = g_expand(ptr<uint16_t>(z), ptr<uint16_t>(b), ptr<int64_t>(offsets), ptr<int32_t>(strides), ptr<uint16_t>(y),
-                          ptr<int32_t>(indptr), ptr<int32_t>(slots), ptr<int32_t>(tokens), ptr<int32_t>(ranks),
-                          ptr<float>(scales), ptr<int32_t>(bounds), ptr<int32_t>(count), slots->numel(), m, n, y->stride(0),
-                          int32_t(slices), z->size(1) / slices, int32_t(blocks), int32_t(threads), stream);
+  const int rc = unlocked([&] {
+    return g_expand(ptr<uint16_t>(z), ptr<uint16_t>(b), ptr<int64_t>(offsets), ptr<int32_t>(strides), ptr<uint16_t>(y),
+                    ptr<int32_t>(indptr), ptr<int32_t>(slots), ptr<int32_t>(tokens), ptr<int32_t>(ranks),
+                    ptr<float>(scales), ptr<int32_t>(bounds), ptr<int32_t>(count), slots->numel(), m, n, y->stride(0),
+                    int32_t(slices), z->size(1) / slices, int32_t(blocks), int32_t(threads), stream);
+  });
   if (rc == LF_EINVAL) return decline();
   if (rc != LF_OK) {
     PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in row_expand");
@@ -526,7 +548,9 @@ PyObject* dequant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!current(dev, &stream)) return decline();
   at::Tensor out = at::empty({n, k}, s->options().dtype(at::kBFloat16));
   if (!on_gpu(out)) return decline();
-  const int rc = g_dequant(ptr<uint8_t>(q), ptr<float>(s), ptr<float>(c), static_cast<uint16_t*>(out.data_ptr()), size, stream);
+  const int rc = unlocked([&] {
+    return g_dequant(ptr<uint8_t>(q), ptr<float>(s), ptr<float>(c), static_cast<uint16_t*>(out.data_ptr()), size, stream);
+  });
   if (rc == LF_EINVAL) return decline();
   if (rc != LF_OK) {
     PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in dequantize_nf4");
@@ -564,13 +588,12 @@ PyObject* dequant_nested(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!current(dev, &stream)) return decline();
   at::Tensor out = at::empty({n, k}, code->options().dtype(at::kBFloat16));
   if (!on_gpu(out)) return decline();
-  int rc = LF_OK;
   int32_t canonical = 0;
   uint16_t* dst = static_cast<uint16_t*>(out.data_ptr());
-  Py_BEGIN_ALLOW_THREADS
-  rc = g_dequant_dq(ptr<uint8_t>(q), w.absmax_q, w.absmax2, w.code2, w.offset, w.dq_block, ptr<float>(code), dst, size,
-                    &canonical, stream);
-  Py_END_ALLOW_THREADS
+  const int rc = unlocked([&] {
+    return g_dequant_dq(ptr<uint8_t>(q), w.absmax_q, w.absmax2, w.code2, w.offset, w.dq_block, ptr<float>(code), dst, size,
+                        &canonical, stream);
+  });
   if (rc == LF_EINVAL || (rc == LF_OK && !canonical)) return decline();
   if (rc != LF_OK) {
     PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in dequantize_nf4_nested");

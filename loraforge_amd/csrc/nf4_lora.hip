@@ -3,6 +3,7 @@
 // larger batch that the prefill tiles would not spread over the chip) and the
 // prefill GEMM.
 #include <algorithm>
+#include <mutex>
 
 #include "nf4_common.h"
 #include "../../include/loraforge_amd.h"
@@ -33,6 +34,15 @@ int launch_decode_wide(const uint16_t* x, int64_t m, int64_t x_stride, const lf_
                        const lf_lora* lora, uint16_t* y, int64_t y_stride, void* workspace, int64_t workspace_bytes,
                        bool exact, bool swiglu, bool withhold, void* stream);
 constexpr int64_t kDecodeMaxTokens = 64;
+
+// Held while a call's launches go out, so that they stay together on the stream:
+// the launches of one call hand z rows, rebuilt scales and the call's tag to each
+// other through the workspace, and threads that share a stream share its cached
+// workspace.
+std::mutex& launch_lock(const void* workspace) {
+  static std::mutex locks[64];
+  return locks[(reinterpret_cast<uintptr_t>(workspace) >> 12) % 64];
+}
 
 double prefill_us(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu);
 
@@ -130,6 +140,7 @@ extern "C" int lf_nf4_lora_linear(const uint16_t* x, int64_t m, int64_t x_stride
     LF_REQUIRE(lf::aligned16(lora->a_store) && lf::aligned16(lora->b_store), "A/B stores must be 16-byte aligned");
   }
   const bool exact = (flags & LF_EXACT_WEIGHTS) != 0;
+  std::lock_guard<std::mutex> together(lf::launch_lock(workspace));
   // Above 8 tokens (2 at N >= 8192, 16 at K > 8192): the wide decode kernel
   // (one launch, base linear with or without LoRA and the SwiGLU output),
   // unless the prefill GEMM is forced or cheaper, or the shape is outside the
@@ -207,6 +218,7 @@ extern "C" int lf_lora_apply(const uint16_t* x, int64_t m, int64_t x_stride, int
   shape.n = n;
   shape.k = k;
   const bool withhold = (flags & LF_TEST_WITHHOLD_PARTIALS) != 0;
+  std::lock_guard<std::mutex> together(lf::launch_lock(workspace));
   // Above 64 tokens, where it is cheaper: shrink and expand as two launches
   // over all tokens whose z rows the workspace holds. A workspace that holds
   // fewer than 128 tokens' rows takes the launches per 64 tokens below.

@@ -6,7 +6,10 @@ the second call of a shape runs natively, a call with ``workspace=`` or with
 the native path switched off runs in Python.
 """
 
+import contextlib
+import ctypes
 import dataclasses
+import threading
 
 import pytest
 import torch
@@ -32,6 +35,16 @@ class _Declines:
 
     def __getattr__(self, name):
         return lambda *args: None
+
+
+@contextlib.contextmanager
+def standing_in(**replaced):
+    """The native call path with other entry points (addresses by name)."""
+    _lib.bind(_lib.binding(), **replaced)
+    try:
+        yield
+    finally:
+        _lib.bind(_lib.binding())
 
 
 def both(monkeypatch, call):
@@ -139,3 +152,72 @@ def test_refusals_are_the_python_path_s(device):
     with pytest.raises(ValueError, match="16-entry"):
         dequantize_nf4(q, st.absmax, st.code[:8], (256, 512))
     assert torch.equal(nf4_lora_linear(x, q, st, lora=lora), good)
+
+
+def operators(device):
+    """Each operator with a native path, as a function that says whether that path took the call."""
+    case = _cases.fused_case(4, 256, 512, ranks=(8, 4), seed=461)
+    x, q, st, lora, _ = to_device(case, device)
+    y = torch.zeros(4, 256, dtype=torch.bfloat16, device=device)
+    nested = _cases.fused_case(4, 256, 512, ranks=(8,), double_quant=True, seed=462)
+    _, q2, st2, _, _ = to_device(nested, device)
+    c = _cases.c2_case(seed=463, tokens=24, k=512, n=256, adapters=4)
+    t = lambda a: torch.from_numpy(a.view("int16") if a.dtype == "uint16" else a).to(device)
+    bf = lambda a: t(a).view(torch.bfloat16)
+    rx, a, b, z, ry, routes = bf(c["x"]), bf(c["a"]), bf(c["b"]), bf(c["z"]), bf(c["y"]), t(c["routes"])
+    meta = {k: t(v) for k, v in c["meta"].items()}
+    order = ("b_offsets", "b_strides", "ranks", "scales", "segment_indptr", "segment_slots", "token_indices", "slice_offsets",
+             "segment_count")
+    # A first call of each through its Python path: device flags, workspaces.
+    nf4_lora_linear(x, q, st, lora=lora)
+    lora_apply(x, y, lora)
+    row_shrink(rx, a, z, routes, meta["ranks"], max_rank=16)
+    row_expand(z, b, ry, **meta)
+    dequantize_nf4(q, st.absmax, st.code, (256, 512))
+    dequantize_nf4_nested(q2, st2)
+    native = _lib.binding()
+    return {
+        "lf_nf4_lora_linear": lambda: native.linear(x, q, st, None, None, lora, None, False, False, 0),
+        "lf_lora_apply": lambda: native.apply(x, y, lora),
+        "lf_row_shrink": lambda: native.shrink(rx, a, z, routes, meta["ranks"], 1, 16),
+        "lf_row_expand": lambda: native.expand(z, b, ry, *(meta[k] for k in order), None, 256),
+        "lf_nf4_dequant": lambda: native.dequant(q, st.absmax, st.code, (256, 512)),
+        "lf_nf4_dequant_dq_checked": lambda: native.dequant_nested(q2, st2),
+    }
+
+
+def test_library_calls_run_without_the_gil(device):
+    """In the library's place stands PyGILState_Check, whose answer reads as a status: 0 (no GIL held)
+    is LF_OK, 1 LF_EINVAL, on which the native path declines. (The checked dequantisation then finds
+    its unset answer not canonical and declines too.)"""
+    check = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    for name, call in operators(device).items():
+        assert call() is not None, name
+        with standing_in(**{name: check}):
+            assert (call() is not None) or name == "lf_nf4_dequant_dq_checked", name
+
+
+def test_threads_on_one_stream_share_its_workspace(device):
+    """Calls of several launches that hand z rows over in the cached workspace, from threads on one
+    stream: each keeps its launches together."""
+    cases = [_cases.fused_case(m, 512, 2048, ranks=(16, 8, 4), seed=470 + m) for m in (200, 270, 330)]
+    jobs = []
+    for case in cases:
+        x, q, st, lora, _ = to_device(case, device)
+        base = torch.randn(case["m"], 512, device=device).bfloat16()
+        want = lora_apply(x, base.clone(), lora)
+        jobs.append((x, base, lora, want))
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(x, base, lora, want):
+        for _ in range(100):
+            if not torch.equal(lora_apply(x, base.clone(), lora), want):
+                wrong.append(x.shape)
+
+    threads = [threading.Thread(target=work, args=job) for job in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
