@@ -61,7 +61,8 @@ int lf_nf4_dequant_dq(const uint8_t* qweight, const uint8_t* absmax_q, const flo
 /* The same, with the canonical-codebook check (ops/nf4.py:120-141) made by the
  * kernel: *canonical says whether `code` holds the canonical 16 values (if
  * not, `out` is not to be used). Waits until the kernel has started, so not
- * under graph capture (LF_EINVAL). */
+ * under graph capture (LF_EINVAL). At most 256 such calls at a time, over all
+ * threads and streams (LF_EINVAL; the unchecked call has no such limit). */
 int lf_nf4_dequant_dq_checked(const uint8_t* qweight, const uint8_t* absmax_q, const float* absmax2,
                               const float* code2, const float* offset, int64_t dq_block, const float* code,
                               uint16_t* out, int64_t numel, int32_t* canonical, void* stream);

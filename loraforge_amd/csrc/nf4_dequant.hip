@@ -16,11 +16,11 @@
 // aligned, or an output that is not 16-byte aligned (a contiguous view at an
 // odd offset, which the reference accepts), take the same kernel with byte
 // loads and 2-byte stores.
-#include <atomic>
 #include <chrono>
 #include <mutex>
 
 #include "nf4_common.h"
+#include "verdict_words.h"
 #include "../../include/loraforge_amd.h"
 
 namespace lf {
@@ -76,18 +76,15 @@ __constant__ const float kCanonical[16] = {
     1.0f,
 };
 
-// A checked call's answer: its ticket, and whether the codebook is canonical,
-// in one word of host memory (verdict null: unchecked).
-struct Verdict {
-  uint64_t* word;
-  uint32_t ticket;
-};
+// A checked call's answer in a word of host memory: kAnswered, plus 1 for the
+// canonical codebook (word null: unchecked).
+constexpr uint32_t kAnswered = 2;
 
 template <bool kDouble, bool kAligned, int kSteps>
 __global__ __launch_bounds__(kThreads) void nf4_dequant_kernel(const uint8_t* __restrict__ packed,
                                                                ScaleSource src, const float* __restrict__ code,
                                                                uint16_t* __restrict__ out, int64_t ndwords,
-                                                               Verdict verdict) {
+                                                               uint32_t* verdict) {
   __shared__ float table[16];
   __shared__ float code2[kDouble ? 256 : 1];
   // Packed bytes are requested first; the codebook is staged while they travel.
@@ -102,11 +99,10 @@ __global__ __launch_bounds__(kThreads) void nf4_dequant_kernel(const uint8_t* __
   if (threadIdx.x < 16) table[threadIdx.x] = code[threadIdx.x];
   if constexpr (kDouble) code2[threadIdx.x] = src.code2[threadIdx.x];
   __syncthreads();
-  if (kDouble && verdict.word && blockIdx.x == 0 && threadIdx.x < 64) {
+  if (kDouble && verdict && blockIdx.x == 0 && threadIdx.x < 64) {
     const uint64_t same = __ballot(threadIdx.x >= 16 || table[threadIdx.x & 15] == kCanonical[threadIdx.x & 15]);
     if (threadIdx.x == 0)
-      __hip_atomic_store(verdict.word, (uint64_t(verdict.ticket) << 1) | (same == ~uint64_t(0) ? 1u : 0u), __ATOMIC_RELEASE,
-                         __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(verdict, kAnswered | (same == ~uint64_t(0) ? 1u : 0u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 #pragma unroll
   for (int s = 0; s < kSteps; ++s) {
@@ -132,7 +128,7 @@ __global__ __launch_bounds__(kThreads) void dq_scales_kernel(ScaleSource src, fl
 }
 
 int launch_dequant(const uint8_t* qweight, const ScaleSource& src, const float* code, uint16_t* out,
-                   int64_t numel, void* stream, Verdict verdict = Verdict{nullptr, 0}) {
+                   int64_t numel, void* stream, uint32_t* verdict = nullptr) {
   LF_REQUIRE(numel > 0 && numel % (kNf4Block * kNf4Block) == 0,
              "element count must be a positive multiple of 4096");
   LF_REQUIRE(qweight && code && out, "null pointer argument");
@@ -155,12 +151,11 @@ int launch_dequant(const uint8_t* qweight, const ScaleSource& src, const float* 
   return kOk;
 }
 
-// Words for the answers of checked calls in flight (one per call, in turn).
-// Pinned host memory of one page, kept until the process ends.
-constexpr uint32_t kVerdicts = 256;
-std::mutex g_verdict_lock;
-uint64_t* g_verdicts = nullptr;
-std::atomic<uint32_t> g_ticket{0};
+// Words for the answers of checked calls, one for each call in flight. Pinned
+// host memory of one page, kept until the process ends.
+VerdictWords g_words;
+std::mutex g_page_lock;
+uint32_t* g_page = nullptr;
 
 }  // namespace
 }  // namespace lf
@@ -175,40 +170,41 @@ extern "C" int lf_nf4_dequant_dq_checked(const uint8_t* qweight, const uint8_t* 
   LF_HIP(hipStreamIsCapturing(s, &capture));
   LF_REQUIRE(capture == hipStreamCaptureStatusNone, "a checked call waits for its answer: not under graph capture");
   {
-    std::lock_guard<std::mutex> guard(lf::g_verdict_lock);
-    if (lf::g_verdicts == nullptr) {
+    std::lock_guard<std::mutex> guard(lf::g_page_lock);
+    if (lf::g_page == nullptr) {
       void* page = nullptr;
-      LF_HIP(hipHostMalloc(&page, lf::kVerdicts * sizeof(uint64_t), hipHostMallocPortable));
-      for (uint32_t i = 0; i < lf::kVerdicts; ++i) static_cast<uint64_t*>(page)[i] = 0;
-      lf::g_verdicts = static_cast<uint64_t*>(page);
+      LF_HIP(hipHostMalloc(&page, lf::VerdictWords::kWords * sizeof(uint32_t), hipHostMallocPortable));
+      lf::g_page = static_cast<uint32_t*>(page);
     }
   }
-  // (Ticket 0 is what an unused word holds.)
-  uint32_t ticket;
-  do ticket = lf::g_ticket.fetch_add(1, std::memory_order_relaxed) + 1;
-  while (ticket == 0);
-  uint64_t* word = lf::g_verdicts + ticket % lf::kVerdicts;
+  const int index = lf::g_words.take();
+  LF_REQUIRE(index >= 0, "%d checked calls in flight already", lf::VerdictWords::kWords);
+  uint32_t* word = lf::g_page + index;
+  __atomic_store_n(word, 0u, __ATOMIC_RELAXED);
+  // Nothing writes the word once the call is answered, or its kernel never
+  // launched or finished: then it goes back.
+  const auto returned = [&](int rc) {
+    lf::g_words.give(index);
+    return rc;
+  };
   void* device_word = nullptr;
-  LF_HIP(hipHostGetDevicePointer(&device_word, word, 0));
+  if (const hipError_t err = hipHostGetDevicePointer(&device_word, word, 0); err != hipSuccess)
+    return returned(lf::hip_status(err, "hipHostGetDevicePointer"));
   lf::ScaleSource src{nullptr, absmax_q, absmax2, code2, offset, int(dq_block)};
-  const int rc = lf::launch_dequant(qweight, src, code, out, numel, stream,
-                                    lf::Verdict{static_cast<uint64_t*>(device_word), ticket});
-  if (rc != lf::kOk) return rc;
+  const int rc = lf::launch_dequant(qweight, src, code, out, numel, stream, static_cast<uint32_t*>(device_word));
+  if (rc != lf::kOk) return returned(rc);
   // The answer comes as the kernel starts: a short look for it, then the
   // stream's own wait (work ahead of the kernel, or an error).
-  auto answered = [&](uint64_t* v) {
-    *v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
-    return uint32_t(*v >> 1) == ticket;
-  };
-  uint64_t v = 0;
   const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
-  while (!answered(&v)) {
+  uint32_t answer;
+  while ((answer = __atomic_load_n(word, __ATOMIC_ACQUIRE)) == 0) {
     if (std::chrono::steady_clock::now() < until) continue;
-    LF_HIP(hipStreamSynchronize(s));
-    if (!answered(&v)) return lf::fail(lf::kHip, "the codebook check gave no answer");
+    LF_HIP(hipStreamSynchronize(s));  // (failed: the kernel may still run, the word stays taken)
+    if ((answer = __atomic_load_n(word, __ATOMIC_ACQUIRE)) == 0)
+      return returned(lf::fail(lf::kHip, "the codebook check gave no answer"));
   }
-  *canonical = int32_t(v & 1);
-  return lf::kOk;
+  *canonical = int32_t(answer & 1);
+  return returned(lf::kOk);
 }
 
 extern "C" int lf_nf4_dequant(const uint8_t* qweight, const float* scales, const float* code, uint16_t* out,
