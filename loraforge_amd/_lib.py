@@ -192,6 +192,7 @@ _BOUND = (
     "lf_row_expand",
     "lf_nf4_dequant",
     "lf_nf4_dequant_dq_checked",
+    "lf_last_error",
 )
 
 

@@ -16,6 +16,8 @@
 // module binds to whatever build of the library the process loaded.
 #include <Python.h>
 
+#include <cstring>
+
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -33,6 +35,7 @@ decltype(&lf_row_shrink_workspace_size) g_shrink_ws;
 decltype(&lf_row_expand) g_expand;
 decltype(&lf_nf4_dequant) g_dequant;
 decltype(&lf_nf4_dequant_dq_checked) g_dequant_dq;
+decltype(&lf_last_error) g_last_error;
 
 PyObject* g_raw_stream;   // torch._C._cuda_getCurrentRawStream
 PyObject* g_get_device;   // torch._C._cuda_getDevice
@@ -60,6 +63,14 @@ struct Ref {
 PyObject* decline() {
   PyErr_Clear();
   Py_RETURN_NONE;
+}
+
+// A HIP error of a library call, with the library's text (as _lib.check raises it).
+PyObject* failed() {
+  const char* text = g_last_error();
+  Ref message(PyUnicode_DecodeUTF8(text, Py_ssize_t(strlen(text)), "replace"));
+  if (message) PyErr_SetObject(PyExc_RuntimeError, message.p);
+  return nullptr;
 }
 
 // The tensor behind a Python object if it is an ordinary dense GPU tensor
@@ -385,10 +396,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                     int32_t(flags) | (exact ? LF_EXACT_WEIGHTS : 0) | (swiglu ? LF_SWIGLU_OUTPUT : 0), stream);
   });
   if (rc == LF_EINVAL) return decline();  // (nothing was launched; the Python path raises the message)
-  if (rc != LF_OK) {
-    PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in nf4_lora_linear");
-    return nullptr;
-  }
+  if (rc != LF_OK) return failed();
   if (py_out != Py_None) {
     Py_INCREF(py_out);
     return py_out;
@@ -422,10 +430,7 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                    ws.numel(), 0, stream);
   });
   if (rc == LF_EINVAL) return decline();
-  if (rc != LF_OK) {
-    PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in lora_apply");
-    return nullptr;
-  }
+  if (rc != LF_OK) return failed();
   Py_INCREF(args[1]);
   return args[1];
 }
@@ -464,10 +469,7 @@ PyObject* shrink(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                     need ? ws.data_ptr() : nullptr, need ? ws.numel() : 0, 0, stream);
   });
   if (rc == LF_EINVAL) return decline();
-  if (rc != LF_OK) {
-    PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in row_shrink");
-    return nullptr;
-  }
+  if (rc != LF_OK) return failed();
   Py_RETURN_TRUE;
 }
 
@@ -519,10 +521,7 @@ PyObject* expand(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                     int32_t(slices), z->size(1) / slices, int32_t(blocks), int32_t(threads), stream);
   });
   if (rc == LF_EINVAL) return decline();
-  if (rc != LF_OK) {
-    PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in row_expand");
-    return nullptr;
-  }
+  if (rc != LF_OK) return failed();
   Py_RETURN_TRUE;
 }
 
@@ -552,10 +551,7 @@ PyObject* dequant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return g_dequant(ptr<uint8_t>(q), ptr<float>(s), ptr<float>(c), static_cast<uint16_t*>(out.data_ptr()), size, stream);
   });
   if (rc == LF_EINVAL) return decline();
-  if (rc != LF_OK) {
-    PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in dequantize_nf4");
-    return nullptr;
-  }
+  if (rc != LF_OK) return failed();
   return THPVariable_Wrap(out);
 }
 
@@ -595,10 +591,7 @@ PyObject* dequant_nested(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                         &canonical, stream);
   });
   if (rc == LF_EINVAL || (rc == LF_OK && !canonical)) return decline();
-  if (rc != LF_OK) {
-    PyErr_SetString(PyExc_RuntimeError, "loraforge_amd: HIP runtime error in dequantize_nf4_nested");
-    return nullptr;
-  }
+  if (rc != LF_OK) return failed();
   return THPVariable_Wrap(out);
 }
 
@@ -608,12 +601,13 @@ PyObject* init(PyObject*, PyObject* args) {
   if (!PyArg_ParseTuple(args, "O!OOO!O!O!", &PyTuple_Type, &addresses, &raw, &dev, &PyDict_Type, &arch, &PyDict_Type, &ws,
                         &PyDict_Type, &cus))
     return nullptr;
-  void* a[8];
-  if (PyTuple_GET_SIZE(addresses) != 8) {
-    PyErr_SetString(PyExc_ValueError, "eight entry points expected");
+  constexpr int kEntries = 9;
+  void* a[kEntries];
+  if (PyTuple_GET_SIZE(addresses) != kEntries) {
+    PyErr_SetString(PyExc_ValueError, "nine entry points expected");
     return nullptr;
   }
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < kEntries; ++i)
     if (!(a[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(addresses, i)))) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null entry point");
       return nullptr;
@@ -626,6 +620,7 @@ PyObject* init(PyObject*, PyObject* args) {
   g_expand = reinterpret_cast<decltype(g_expand)>(a[5]);
   g_dequant = reinterpret_cast<decltype(g_dequant)>(a[6]);
   g_dequant_dq = reinterpret_cast<decltype(g_dequant_dq)>(a[7]);
+  g_last_error = reinterpret_cast<decltype(g_last_error)>(a[8]);
 #define INTERN(n) \
   if (!s_##n && !(s_##n = PyUnicode_InternFromString(#n))) return nullptr;
   NAMES(INTERN)

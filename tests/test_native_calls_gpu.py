@@ -221,3 +221,14 @@ def test_threads_on_one_stream_share_its_workspace(device):
     for t in threads:
         t.join()
     assert not wrong
+
+
+def test_hip_errors_carry_the_library_s_text(device):
+    """A library call that fails with a HIP error raises lf_last_error()'s text, as the Python path does."""
+    status = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: _lib.LF_EHIP)
+    text = ctypes.CFUNCTYPE(ctypes.c_char_p)(lambda: b"hipLaunchKernel failed: out of memory")
+    address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
+    for name, call in operators(device).items():
+        with standing_in(**{name: address(status), "lf_last_error": address(text)}):
+            with pytest.raises(RuntimeError, match="hipLaunchKernel failed: out of memory"):
+                call()
