@@ -200,11 +200,13 @@ def bind(module, **replaced) -> None:
     """Hand the native call path its entry points (``replaced``: addresses that stand in for some)."""
     import torch
 
+    from .ops.fused import LoraBatch
+
     stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda index: torch.cuda.current_stream(index).cuda_stream)
     device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
     lib = library()
     addresses = tuple(replaced.get(name) or ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _BOUND)
-    module.init(addresses, stream, device, ARCH_OK, WORKSPACES, COMPUTE_UNITS)
+    module.init(addresses, stream, device, ARCH_OK, WORKSPACES, COMPUTE_UNITS, LoraBatch)
 
 
 def binding():

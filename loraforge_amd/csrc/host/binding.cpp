@@ -42,6 +42,7 @@ PyObject* g_get_device;   // torch._C._cuda_getDevice
 PyObject* g_arch_ok;      // device index -> whether the kernels run there
 PyObject* g_workspaces;   // the operators' workspace cache
 PyObject* g_multi_cus;    // device index -> compute units
+PyObject* g_lora_batch;   // ops.fused.LoraBatch
 
 #define NAMES(X)                                                                                                     \
   X(absmax) X(shape) X(code) X(blocksize) X(quant_type) X(offset) X(state2) X(nested) X(_lf_prepared_scales)         \
@@ -169,6 +170,7 @@ T* ptr(const at::Tensor* t) {
 }
 
 // The C descriptor of a LoraBatch (its fields as ops.fused._lora_struct checks them).
+// A subclass or another object may have a num_slices of its own: the Python path's.
 struct LoraArg {
   lf_lora d{};
   int slices = 1;
@@ -178,6 +180,7 @@ struct LoraArg {
     for (PyObject* o : held) Py_XDECREF(o);
   }
   bool take(PyObject* b, int64_t m, const at::Device& dev) {
+    if (reinterpret_cast<PyObject*>(Py_TYPE(b)) != g_lora_batch) return false;
     PyObject* names[10] = {s_a_store, s_a_offsets, s_b_store, s_b_offsets, s_b_strides,
                            s_ranks,   s_scales,    s_token_slots, s_slice_offsets, s_max_rank};
     for (int i = 0; i < 10; ++i)
@@ -595,11 +598,11 @@ PyObject* dequant_nested(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return THPVariable_Wrap(out);
 }
 
-// init(addresses, raw_stream, get_device, arch_ok, workspaces, compute_units)
+// init(addresses, raw_stream, get_device, arch_ok, workspaces, compute_units, lora_batch)
 PyObject* init(PyObject*, PyObject* args) {
-  PyObject *addresses, *raw, *dev, *arch, *ws, *cus;
-  if (!PyArg_ParseTuple(args, "O!OOO!O!O!", &PyTuple_Type, &addresses, &raw, &dev, &PyDict_Type, &arch, &PyDict_Type, &ws,
-                        &PyDict_Type, &cus))
+  PyObject *addresses, *raw, *dev, *arch, *ws, *cus, *batch;
+  if (!PyArg_ParseTuple(args, "O!OOO!O!O!O!", &PyTuple_Type, &addresses, &raw, &dev, &PyDict_Type, &arch, &PyDict_Type, &ws,
+                        &PyDict_Type, &cus, &PyType_Type, &batch))
     return nullptr;
   constexpr int kEntries = 9;
   void* a[kEntries];
@@ -625,9 +628,9 @@ PyObject* init(PyObject*, PyObject* args) {
   if (!s_##n && !(s_##n = PyUnicode_InternFromString(#n))) return nullptr;
   NAMES(INTERN)
 #undef INTERN
-  PyObject** slot[5] = {&g_raw_stream, &g_get_device, &g_arch_ok, &g_workspaces, &g_multi_cus};
-  PyObject* value[5] = {raw, dev, arch, ws, cus};
-  for (int i = 0; i < 5; ++i) {
+  PyObject** slot[6] = {&g_raw_stream, &g_get_device, &g_arch_ok, &g_workspaces, &g_multi_cus, &g_lora_batch};
+  PyObject* value[6] = {raw, dev, arch, ws, cus, batch};
+  for (int i = 0; i < 6; ++i) {
     Py_INCREF(value[i]);
     Py_XDECREF(*slot[i]);
     *slot[i] = value[i];

@@ -10,12 +10,14 @@ import contextlib
 import ctypes
 import dataclasses
 import threading
+import types
 
 import pytest
 import torch
 
 from loraforge_amd import _lib
 from loraforge_amd.ops import (
+    LoraBatch,
     dequantize_nf4,
     dequantize_nf4_nested,
     lora_apply,
@@ -226,9 +228,33 @@ def test_threads_on_one_stream_share_its_workspace(device):
 def test_hip_errors_carry_the_library_s_text(device):
     """A library call that fails with a HIP error raises lf_last_error()'s text, as the Python path does."""
     status = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: _lib.LF_EHIP)
-    text = ctypes.CFUNCTYPE(ctypes.c_char_p)(lambda: b"hipLaunchKernel failed: out of memory")
+    words = ctypes.create_string_buffer(b"hipLaunchKernel failed: out of memory")
+    text = ctypes.CFUNCTYPE(ctypes.c_void_p)(lambda: ctypes.addressof(words))
     address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
     for name, call in operators(device).items():
         with standing_in(**{name: address(status), "lf_last_error": address(text)}):
             with pytest.raises(RuntimeError, match="hipLaunchKernel failed: out of memory"):
                 call()
+
+
+def test_other_batches_go_the_python_way(device):
+    """The native path reads LoraBatch itself; an object with a num_slices of its own, or without one, is
+    served or refused by the Python path."""
+
+    class Disagreeing(LoraBatch):
+        num_slices = 2
+
+    case = _cases.fused_case(4, 256, 512, ranks=(8, 4), seed=465)
+    x, q, st, lora, _ = to_device(case, device)
+    want = nf4_lora_linear(x, q, st, lora=lora)
+    fields = {f.name: getattr(lora, f.name) for f in dataclasses.fields(lora)}
+    same = type("Same", (LoraBatch,), {})(**fields)
+    assert torch.equal(nf4_lora_linear(x, q, st, lora=same), want)
+    for _ in range(2):
+        with pytest.raises(ValueError, match="slice_offsets length disagrees"):
+            nf4_lora_linear(x, q, st, lora=Disagreeing(**fields))
+        with pytest.raises(ValueError, match="slice_offsets length disagrees"):
+            lora_apply(x, torch.zeros(4, 256, dtype=torch.bfloat16, device=device), Disagreeing(**fields))
+        with pytest.raises(AttributeError, match="num_slices"):
+            nf4_lora_linear(x, q, st, lora=types.SimpleNamespace(**fields))
+    assert torch.equal(nf4_lora_linear(x, q, st, lora=lora), want)
