@@ -234,6 +234,22 @@ int lf_nf4_lora_linear(const uint16_t* x, int64_t m, int64_t x_stride, const lf_
                        const uint16_t* bias, const lf_lora* lora, uint16_t* y, int64_t y_stride,
                        void* workspace, int64_t workspace_bytes, int32_t flags, void* stream);
 
+/* The plan that lf_nf4_lora_linear takes for a call of this size on the current
+ * device (an MI355X where there is none): host arithmetic, nothing is launched.
+ * num_slices 0: without adapters; num_slots as in lf_lora; flags as above. */
+#define LF_KERNEL_DECODE 0        /* narrow decode kernel */
+#define LF_KERNEL_DECODE_WIDE 1   /* wide decode kernel over all tokens */
+#define LF_KERNEL_DECODE_CHUNKS 2 /* decode kernels per 64 tokens */
+#define LF_KERNEL_PREFILL 3
+typedef struct lf_plan {
+  int32_t kernel;
+  int32_t tile_rows; /* prefill: tokens per tile */
+  int32_t z_parts;   /* prefill with adapters: z producers per tile, ... */
+  int32_t z_launch;  /* ... and whether they have a launch of their own */
+} lf_plan;
+int lf_nf4_lora_plan(int64_t m, int64_t n, int64_t k, int32_t num_slices, int32_t max_rank, int32_t num_slots,
+                     int32_t flags, lf_plan* plan);
+
 /* LoRA-only update of existing bf16 outputs, in one launch per 64 tokens or,
  * above 64 tokens over 1..16 slots (num_slots) where cheaper, in two launches
  * over all tokens whose z rows the workspace holds:

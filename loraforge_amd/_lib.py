@@ -24,6 +24,7 @@ LF_SWIGLU_OUTPUT = 2
 LF_PLAN_DECODE_CHUNKS = 4
 LF_PLAN_PREFILL = 8
 LF_TEST_WITHHOLD_PARTIALS = 0x100
+LF_KERNEL_DECODE, LF_KERNEL_DECODE_WIDE, LF_KERNEL_DECODE_CHUNKS, LF_KERNEL_PREFILL = range(4)
 NOALLOC_SCRATCH_BYTES = 8 * 1024 * 1024
 ABI_VERSION = 4
 
@@ -74,6 +75,10 @@ class Lora(ctypes.Structure):
         ("max_rank", c_int32),
         ("num_slots", c_int32),
     ]
+
+
+class Plan(ctypes.Structure):
+    _fields_ = [("kernel", c_int32), ("tile_rows", c_int32), ("z_parts", c_int32), ("z_launch", c_int32)]
 
 
 _PROTOTYPES = {
@@ -147,6 +152,10 @@ _PROTOTYPES = {
         ctypes.c_int,
         [c_void_p, c_int64, c_int64, c_int64, c_int64, ctypes.POINTER(Lora), c_void_p, c_int64, c_void_p, c_int64,
          c_int32, c_void_p],
+    ),
+    "lf_nf4_lora_plan": (
+        ctypes.c_int,
+        [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, ctypes.POINTER(Plan)],
     ),
     "lf_nf4_lora_status": (ctypes.c_int, [c_void_p, c_void_p, ctypes.POINTER(c_int32)]),
     "lf_swiglu": (ctypes.c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p]),

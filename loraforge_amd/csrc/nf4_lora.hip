@@ -45,6 +45,7 @@ std::mutex& launch_lock(const void* workspace) {
 }
 
 double prefill_us(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu);
+void prefill_tiles(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu, lf_plan* plan);
 
 // Whether the wide decode kernel (32 rows x 32 tokens per workgroup over the
 // whole K) serves M > 64 tokens faster than the prefill GEMM (prefill_us):
@@ -70,6 +71,22 @@ bool decode_chunks_cheaper(int64_t m, int64_t n, int64_t k, const lf_lora* lora,
   const int64_t chunks = (m + kDecodeMaxTokens - 1) / kDecodeMaxTokens;
   return double(chunks) * chunk_us < prefill_us(m, n, k, lora, swiglu);
 }
+
+// The kernel of a call. Above 8 tokens (2 at N >= 8192, 16 at K > 8192): the wide
+// decode kernel (one launch, base linear with or without LoRA and the SwiGLU
+// output), unless the prefill GEMM is forced or cheaper, or the shape is outside
+// the kernel's range.
+int kernel_of(int64_t m, int64_t n, int64_t k, const lf_lora* lora, int32_t flags) {
+  const bool swiglu = (flags & LF_SWIGLU_OUTPUT) != 0;
+  if (decode_wide_fits(m, n, k, lora) && !(flags & LF_PLAN_PREFILL) &&
+      (m <= kDecodeMaxTokens || (flags & LF_PLAN_DECODE_CHUNKS) || wide_cheaper(m, n, k, lora, swiglu)))
+    return LF_KERNEL_DECODE_WIDE;
+  if (m <= kDecodeMaxTokens) return LF_KERNEL_DECODE;
+  if (flags & LF_PLAN_DECODE_CHUNKS) return LF_KERNEL_DECODE_CHUNKS;
+  if (flags & LF_PLAN_PREFILL) return LF_KERNEL_PREFILL;
+  return decode_chunks_cheaper(m, n, k, lora, swiglu) ? LF_KERNEL_DECODE_CHUNKS : LF_KERNEL_PREFILL;
+}
+
 // Whether lora_apply's two launches over all tokens are cheaper than a launch
 // of the decode kernel's residual form per 64 tokens. Their time grows with
 // the distinct adapters of a tile (500 tokens x 5120 x 4096, 4 adapters: 31 us
@@ -141,21 +158,14 @@ extern "C" int lf_nf4_lora_linear(const uint16_t* x, int64_t m, int64_t x_stride
   }
   const bool exact = (flags & LF_EXACT_WEIGHTS) != 0;
   std::lock_guard<std::mutex> together(lf::launch_lock(workspace));
-  // Above 8 tokens (2 at N >= 8192, 16 at K > 8192): the wide decode kernel
-  // (one launch, base linear with or without LoRA and the SwiGLU output),
-  // unless the prefill GEMM is forced or cheaper, or the shape is outside the
-  // kernel's range.
-  if (lf::decode_wide_fits(m, n, k, lora) && !(flags & LF_PLAN_PREFILL) &&
-      (m <= lf::kDecodeMaxTokens || (flags & LF_PLAN_DECODE_CHUNKS) || lf::wide_cheaper(m, n, k, lora, swiglu)))
+  const int kernel = lf::kernel_of(m, n, k, lora, flags);
+  if (kernel == LF_KERNEL_DECODE_WIDE)
     return lf::launch_decode_wide(x, m, x_stride, w, bias, lora, y, y_stride, workspace, workspace_bytes, exact,
                                   swiglu, withhold, stream);
-  if (m <= lf::kDecodeMaxTokens)
+  if (kernel == LF_KERNEL_DECODE)
     return lf::launch_decode(x, m, x_stride, w, bias, lora, y, y_stride, workspace, workspace_bytes, exact, swiglu,
                              withhold, stream);
-  bool chunked = false;
-  if (flags & LF_PLAN_DECODE_CHUNKS) chunked = true;
-  else if (!(flags & LF_PLAN_PREFILL)) chunked = lf::decode_chunks_cheaper(m, n, k, lora, swiglu);
-  if (!chunked)
+  if (kernel == LF_KERNEL_PREFILL)
     return lf::launch_nf4_lora_prefill(x, m, x_stride, w, bias, lora, y, y_stride, workspace, workspace_bytes,
                                        swiglu, withhold, stream);
   // 64-token chunks in token order on the caller's stream; each is one decode
@@ -186,6 +196,25 @@ extern "C" int lf_nf4_lora_linear(const uint16_t* x, int64_t m, int64_t x_stride
                                      stream);
     if (rc != lf::kOk) return rc;
   }
+  return lf::kOk;
+}
+
+extern "C" int lf_nf4_lora_plan(int64_t m, int64_t n, int64_t k, int32_t num_slices, int32_t max_rank, int32_t num_slots,
+                                int32_t flags, lf_plan* plan) {
+  LF_REQUIRE(plan != nullptr, "null pointer argument");
+  LF_REQUIRE(m > 0 && m < (int64_t(1) << 31), "token count out of range");
+  LF_REQUIRE(n > 0 && k > 0 && n % 64 == 0 && k % 64 == 0, "weight shape must contain two positive multiples of 64");
+  LF_REQUIRE(n < (int64_t(1) << 28) && k < (int64_t(1) << 28), "weight shape too large");
+  LF_REQUIRE(num_slices >= 0 && num_slices <= 3, "num_slices must be in 1..3, or 0 without adapters");
+  LF_REQUIRE(num_slices == 0 || (max_rank >= 1 && max_rank <= 64), "max_rank must be in 1..64");
+  lf_lora lora{};
+  lora.num_slices = num_slices;
+  lora.max_rank = max_rank;
+  lora.num_slots = num_slots;
+  const lf_lora* adapters = num_slices ? &lora : nullptr;
+  *plan = lf_plan{};
+  plan->kernel = lf::kernel_of(m, n, k, adapters, flags);
+  if (plan->kernel == LF_KERNEL_PREFILL) lf::prefill_tiles(m, n, k, adapters, (flags & LF_SWIGLU_OUTPUT) != 0, plan);
   return lf::kOk;
 }
 

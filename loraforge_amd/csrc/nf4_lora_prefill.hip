@@ -1,6 +1,7 @@
 // Host side of the prefill GEMM (prefill_tile.h): workspace layout, the choice
 // of the tile height and the launch.
 #include <algorithm>
+#include <cmath>
 
 #include "prefill_params.h"
 #include "nf4_common.h"
@@ -26,34 +27,42 @@ constexpr int kMaxZParts = 64;
 // z producers per M-tile inside the GEMM launch: they run first and hold a CU
 // each (one workgroup per CU), which costs nothing where the tiles' last round
 // leaves CUs idle anyway. So they fill that slack (at most 64 per tile, within
-// the flag region). Below 3 a tile (a unit of 16 tokens takes about a tenth of
-// the tile's own time) its consumers would wait for them: 0, a launch of
-// their own.
+// the flag region; 0: none fits).
 int zparts_in_slack(int64_t mtiles, int64_t tiles, int64_t cus) {
   const int64_t rem = tiles % cus;
   const int64_t slack = rem == 0 ? 0 : cus - rem;
-  const int64_t parts = std::min<int64_t>(std::min<int64_t>(kMaxZParts, kMaxFlags / mtiles), slack / mtiles);
-  return parts < 3 ? 0 : int(parts);
+  return int(std::min<int64_t>(std::min<int64_t>(kMaxZParts, kMaxFlags / mtiles), slack / mtiles));
 }
 
 // Tile heights that are built, in 32-token fragments, and the time of a round
-// of such tiles per 4096 of K (us; between a full chip, which runs at a lower
-// clock, and a few tiles). Below 4 fragments the decode of the tile's weights
-// (the same for every height) bounds it instead of the MFMAs.
+// of such tiles per 4096 of K (us) at rounds that are 60 % full (a fuller chip
+// runs at a lower clock: 14 % over the whole range). Below 4 fragments the decode
+// of the tile's weights (the same for every height) bounds it instead of the MFMAs.
 struct TileCost {
   int ri;
   double us;
 };
-constexpr TileCost kTileCosts[] = {{8, 100.0}, {6, 82.0}, {5, 72.0}, {4, 64.0}, {3, 58.0}, {2, 52.0}};
-// What a round takes beside its k-loop: start, rounding and stores, and with
-// LoRA routes, z and B reads and the expand (1024 x 4096 x 1024, rank 16, heights
-// 8 .. 3: 47 / 37 / 35 / 32 / 29 us, of which the k-loop is 25 .. 14).
-double round_us(int ri, bool lora) { return lora ? 9.0 + 1.2 * ri : 4.0 + 0.6 * ri; }
-// A round of z producers of one unit each, one workgroup per CU, in a launch of
-// its own. (More than the kernel's own time, 9-10 us a round at K = 4096: at 5 + rounds x
-// (2.5 + 3 K / 4096) the rule takes the launch in sixteen of four hundred drawn shapes more,
-// and all of them get slower, 1292 x 13824 x 6144 245 -> 266 us.)
-double z_round_us(int64_t k) { return 12.0 + 6.0 * double(k) / 4096.0; }
+constexpr TileCost kTileCosts[] = {{8, 75.0}, {6, 60.0}, {5, 57.0}, {4, 53.0}, {3, 52.0}, {2, 41.5}};
+
+// How a tile of `tokens` tokens may be routed over a pool of adapters: slots
+// among its tokens and among 32 of them, and z units (16 tokens of one slot,
+// half a unit lost to each slot). The host does not know the routes, so a plan
+// is priced for two of them: each slot's tokens together (prompts one after the
+// other), and all slots in turn, the less likely the more tokens a slot has.
+struct Routing {
+  double slots, block, units;
+};
+double units_of(double tokens, double slots) { return std::max(slots, tokens / 16.0 + slots / 2.0); }
+Routing together(double tokens, double m, double pool) {
+  const double slots = std::min({pool, tokens, tokens * pool / m + 1.0});
+  return {slots, 1.0 + std::min(slots - 1.0, 32.0 * pool / m), units_of(tokens, slots)};
+}
+Routing in_turn(double tokens, double pool) {
+  const double slots = pool * tokens / (pool + tokens);
+  return {slots, pool * 32.0 / (pool + 32.0), units_of(tokens, slots)};
+}
+double in_turn_weight(double m, double pool) { return std::min(0.4, 17.0 * pool / m); }
+constexpr int kPoolUnknown = 16;  // adapters of a call that does not say
 
 struct TilePlan {
   int ri;
@@ -63,39 +72,86 @@ struct TilePlan {
   double us;
 };
 
-// The tile height whose rounds of one tile per CU take the least time: 2048 x
-// 11008 x 4096 (43 column tiles) runs in two rounds of 192-token tiles (186 us)
-// instead of two of 256 (208 us), 300 tokens x 24576 (SwiGLU) in one round of
-// 160-token tiles (77 us against 98 us), 4096 x 4096 x 1024 with LoRA in two
-// of 160 tokens (64 us) instead of one of 256, whose z would be a launch of
-// its own.
-TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int slices, int max_rank, bool lora, bool swiglu) {
+// Time of a plan's LoRA call under a routing, us.
+//  - A round's fixed part (start, routes, rounding and stores; without LoRA 5 +
+//    1.2 ri, see tile_plan) and the expand beyond the first slot, per slot and
+//    32-token block.
+//  - Producers in the GEMM launch: a unit takes 2 us and, per 4096 of K, 3.7 us
+//    for each 16 A rows and each 64-row pass (four waves, fragment loads). Their
+//    consumers wait for what does not end within the first round's k-loop (2048 x
+//    11008 x 4096, two slices of rank 32, SwiGLU: 33 producers in the slack of
+//    192-token tiles 244 us, 168 in that of 256-token tiles 219 us; three slices
+//    of rank 64: 408 / 217 us); their loads cost the first tiles about 2 %.
+//  - In a launch of their own (through LDS, one 16-row pass at a time).
+double lora_plan_us(const TilePlan& p, double loop, int64_t cus, int64_t k, int slices, int max_rank, const Routing& r) {
+  const double k4 = double(k) / 4096.0;
+  const double rounds = double((p.tiles + cus - 1) / cus);
+  const int row_tiles = (slices * max_rank + 15) / 16;
+  const double expand = 1.05 * p.ri * std::max(0.0, r.block - 1.0) * (1.0 + 0.1 * ((max_rank + 15) / 16 - 1));
+  const double gemm = rounds * (loop + 7.5 + 2.25 * p.ri + expand);
+  const double serial = std::ceil(r.units / p.zparts);  // units of one producer
+  if (!p.z_launch) return 1.02 * gemm + std::max(0.0, serial * (2.0 + 3.7 * k4 * ((row_tiles + 3) / 4 + row_tiles)) - 0.9 * loop);
+  const int parts = z_row_parts(slices, max_rank);
+  const double groups = double(p.mtiles * p.zparts * parts);
+  const double busy = std::min<double>(r.units, p.zparts) * double(p.mtiles * parts) / double(cus) + 1.0;
+  return gemm + 4.0 + 6.0 * std::ceil(groups / double(cus)) + busy * serial * double((row_tiles + parts - 1) / parts) * (3.0 + 3.0 * k4);
+}
+
+// The tile height, and with LoRA the place of the z producers, that take the
+// least time. (Against the fastest of all heights, with the producers in the slack
+// or in their own launch: 0.4 % slower on average over 5070 drawn calls of 512..4096
+// tokens in prompts, 0.1 % over 2600 of 65..512 tokens in any routing, 28 % at most;
+// the rule that took the slack wherever three producers a tile fit it 1.0 and 0.3 %,
+// up to 87 %, and over a grid of ranks 8..64 and 1..3 slices up to 148 %.)
+TilePlan tile_plan(int64_t m, int64_t n, int64_t k, int slices, int max_rank, bool lora, bool swiglu, int num_slots) {
   const int64_t cus = device_cus();
   const int64_t ntiles = ((swiglu ? n / 2 : n) + (swiglu ? kTileN / 2 : kTileN) - 1) / (swiglu ? kTileN / 2 : kTileN);
+  const double pool = num_slots > 0 ? num_slots : kPoolUnknown;
   TilePlan best{};
   for (const TileCost& c : kTileCosts) {
     TilePlan p{c.ri};
     p.mtiles = (m + 32 * c.ri - 1) / (32 * c.ri);
     if (p.mtiles > kMaxFlags) continue;
     p.tiles = p.mtiles * ntiles;
-    p.us = double((p.tiles + cus - 1) / cus) * (c.us * double(k) / 4096.0 + round_us(c.ri, lora));
-    if (lora) {
-      p.zparts = zparts_in_slack(p.mtiles, p.tiles, cus);
-      p.z_launch = p.zparts == 0;
-      if (p.z_launch) {
-        // A producer per 16 tokens, and two for the units that slot changes add.
-        p.zparts = int(std::max<int64_t>(1, std::min<int64_t>(2 * c.ri + 2, kMaxFlags / p.mtiles)));
-        const int64_t groups = p.mtiles * p.zparts * z_row_parts(slices, max_rank);
-        p.us += z_round_us(k) * double((groups + cus - 1) / cus);
-      }
+    const double rounds = double((p.tiles + cus - 1) / cus);
+    const double full = double(p.tiles) / (rounds * double(cus));
+    const double loop = c.us * (1.0 + 0.14 * (full - 0.6)) * double(k) / 4096.0;
+    if (!lora) {
+      p.us = rounds * (loop + 5.0 + 1.2 * c.ri);
+      if (best.ri == 0 || p.us < best.us) best = p;
+      continue;
     }
-    if (best.ri == 0 || p.us < best.us) best = p;
+    const double tokens = double(std::min<int64_t>(32 * c.ri, m));
+    const Routing routes[2] = {together(tokens, double(m), pool), in_turn(tokens, pool)};
+    const double turn = in_turn_weight(double(m), pool);
+    const int in_launch = zparts_in_slack(p.mtiles, p.tiles, cus);
+    for (const bool launch : {false, true}) {
+      p.z_launch = launch;
+      // (In their own launch: a producer per 16 tokens, and two for the units that slot changes add.)
+      p.zparts = launch ? int(std::max<int64_t>(1, std::min<int64_t>(2 * c.ri + 2, kMaxFlags / p.mtiles))) : in_launch;
+      if (p.zparts == 0) continue;
+      p.us = (1.0 - turn) * lora_plan_us(p, loop, cus, k, slices, max_rank, routes[0]) +
+             turn * lora_plan_us(p, loop, cus, k, slices, max_rank, routes[1]);
+      if (best.ri == 0 || p.us < best.us) best = p;
+    }
   }
   return best;
 }
 
+// Time of a prefill launch for the choice between it and the decode kernels. (A
+// pool counts for at most 64 slots here: of more, few have a token.)
 double prefill_us(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu) {
-  return tile_plan(m, n, k, lora ? lora->num_slices : 1, lora ? lora->max_rank : 1, lora != nullptr, swiglu).us;
+  return tile_plan(m, n, k, lora ? lora->num_slices : 1, lora ? lora->max_rank : 1, lora != nullptr, swiglu,
+                   lora ? std::min(lora->num_slots, 64) : 0)
+      .us;
+}
+
+void prefill_tiles(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu, lf_plan* plan) {
+  const TilePlan p = tile_plan(m, n, k, lora ? lora->num_slices : 1, lora ? lora->max_rank : 1, lora != nullptr, swiglu,
+                               lora ? lora->num_slots : 0);
+  plan->tile_rows = 32 * p.ri;
+  plan->z_parts = p.zparts;
+  plan->z_launch = p.z_launch ? 1 : 0;
 }
 
 int64_t prefill_workspace_bytes(int64_t m, int64_t n, int64_t k, int slices, int) {
@@ -165,7 +221,8 @@ int launch_nf4_lora_prefill(const uint16_t* x, int64_t m, int64_t x_stride, cons
   // SwiGLU output: each tile takes kBN / 2 activation columns (their gate and
   // up rows) and stores 16-byte chunks of them.
   LF_REQUIRE(!swiglu || p.y_vec == 2, "prefill SwiGLU output needs y 16-byte aligned with row stride %% 8 == 0");
-  const TilePlan plan = tile_plan(m, w->n, w->k, slices, lora ? lora->max_rank : 1, lora != nullptr, swiglu);
+  const TilePlan plan = tile_plan(m, w->n, w->k, slices, lora ? lora->max_rank : 1, lora != nullptr, swiglu,
+                                  lora ? lora->num_slots : 0);
   p.tile_rows = 32 * plan.ri;
   p.mtiles = int(plan.mtiles);
   p.zparts = plan.zparts;

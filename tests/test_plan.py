@@ -1,0 +1,44 @@
+"""The kernel and tiles that a fused linear takes (``lf_nf4_lora_plan``: host arithmetic, CPU only)."""
+
+import ctypes
+import math
+
+import pytest
+
+from loraforge_amd import _lib
+
+
+def plan_of(m, n, k, slices=0, rank=1, slots=0, flags=0):
+    plan = _lib.Plan()
+    _lib.check(_lib.library().lf_nf4_lora_plan(m, n, k, slices, rank, slots, flags, ctypes.byref(plan)))
+    return plan
+
+
+@pytest.mark.parametrize("m", [1024, 1500, 2048, 4096])
+@pytest.mark.parametrize("n,k", [(4096, 4096), (11008, 4096), (4096, 11008), (5120, 8192), (24576, 4096)])
+@pytest.mark.parametrize("slices,rank", [(1, 8), (1, 16), (1, 32), (1, 64), (2, 16), (2, 32), (2, 64), (3, 16), (3, 64)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_z_producers_keep_up_with_the_tiles(m, n, k, slices, rank, swiglu):
+    """What z producers inside the GEMM launch take beyond the first round's k-loop, which their tiles
+    wait for, is at most a fifth of all rounds' (nine tenths above 64 A rows a slot; eight prompts of
+    equal length)."""
+    if swiglu and slices != 2:
+        pytest.skip("a SwiGLU output has two slices")
+    plan = plan_of(m, n, k, slices, rank, 8, _lib.LF_PLAN_PREFILL | (_lib.LF_SWIGLU_OUTPUT if swiglu else 0))
+    if plan.z_launch:
+        return
+    units = math.ceil(plan.tile_rows / 16 + 0.5 * (1 + 8 * plan.tile_rows / m))
+    row_tiles = math.ceil(slices * rank / 16)
+    # A unit takes 3.7 us per 4096 of K for each 16 A rows and each pass of 64 of them, the k-loop 10 us per
+    # 32 tokens (and no less than 47 us, for the decode of the weights).
+    z_us = math.ceil(units / plan.z_parts) * 3.7 * (math.ceil(row_tiles / 4) + row_tiles)
+    loop_us = max(47.0, 10.0 * plan.tile_rows / 32)
+    tiles = math.ceil(m / plan.tile_rows) * math.ceil(n / 256)
+    share = 0.2 if row_tiles <= 4 else 0.9
+    assert z_us - loop_us <= share * loop_us * math.ceil(tiles / 256), (plan.tile_rows, plan.z_parts)
+
+
+def test_refusals():
+    for bad in (dict(m=0), dict(n=100), dict(k=0), dict(slices=4), dict(slices=1, rank=65)):
+        with pytest.raises(ValueError):
+            plan_of(**{**dict(m=128, n=256, k=256), **bad})
