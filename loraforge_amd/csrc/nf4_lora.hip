@@ -47,46 +47,72 @@ std::mutex& launch_lock(const void* workspace) {
 double prefill_us(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu);
 void prefill_tiles(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu, lf_plan* plan);
 
-// Whether the wide decode kernel (32 rows x 32 tokens per workgroup over the
-// whole K) serves M > 64 tokens faster than the prefill GEMM (prefill_us):
-// a round of 256 wide workgroups takes 7.5 us per 4096 of K, 8.8 us with LoRA
-// (its per-CU x and weight reads; 256 tokens x 4096: 30 / 40 us against 56 /
-// 65 us on the prefill GEMM, 256 x 11008: 98 us against 67 us).
-bool wide_cheaper(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu) {
+double decode_rounds(int64_t m, int64_t n) {
   const int64_t cus = device_cus();
-  const int64_t wide_groups = ((n / 32 + 7) / 8) * 8 * ((m + 31) / 32);
-  const double wide_us = double((wide_groups + cus - 1) / cus) * (lora ? 8.8 : 7.5) * double(k) / 4096.0;
-  return wide_us < prefill_us(m, n, k, lora, swiglu);
+  const int64_t groups = ((n / 32 + 7) / 8) * 8 * ((m + 31) / 32);
+  return double((groups + cus - 1) / cus);
 }
 
-// Whether M > 64 tokens that the wide kernel does not take are served faster
-// by decode launches over 64-token chunks than by one prefill launch (few
-// tiles leave most of the chip idle; each decode chunk streams W again but
-// uses every CU). A decode launch of 64 tokens streams its weight bytes
-// (packed + fp32 scales) at about 0.8 TB/s, plus about 6 us with LoRA (4096 x
-// 4096: 11.9 us base only, 18.0 us with 32 rank-16 adapters).
-bool decode_chunks_cheaper(int64_t m, int64_t n, int64_t k, const lf_lora* lora, bool swiglu) {
-  const double weight_bytes = double(n) * double(k) * (0.5 + 4.0 / 64.0);
-  const double chunk_us = (lora ? 6.0 : 0.0) + weight_bytes / 0.8e6;
+// What the decode kernels take, us. A call of the wide one: a start and rounds of
+// 256 workgroups (32 rows x 32 tokens over the whole K), each with its own start, x
+// and weight reads and, with LoRA, shrink, z wait and expand. (24576 x 64, 4096
+// tokens: 384 rounds in 911 us; 8192 x 2048, 1024 tokens, three slices of rank 64: 32
+// rounds in 592 us; 14 % rms over 2818 calls with adapters, 7 % over 191 without.)
+double wide_us(int64_t m, int64_t n, int64_t k, const lf_lora* lora) {
+  const double k4 = double(k) / 4096.0;
+  if (!lora) return 2.0 + decode_rounds(m, n) * (2.3 + 5.3 * k4);
+  const double rows = double(lora->num_slices) * lora->max_rank;
+  return 6.3 + decode_rounds(m, n) * (3.1 + 0.062 * rows + (4.8 + 0.024 * rows) * k4);
+}
+// A weight's bytes (packed + fp32 scales) at about 0.8 TB/s, and about 6 us with
+// LoRA (4096 x 4096: 11.9 us base only, 18.0 us with 32 rank-16 adapters).
+double stream_us(int64_t n, int64_t k, const lf_lora* lora) {
+  return (lora ? 6.0 : 0.0) + double(n) * double(k) * (0.5 + 4.0 / 64.0) / 0.8e6;
+}
+// A launch per 64-token chunk, of the wide kernel or the narrow one (14 % rms over
+// 532 calls with adapters).
+double chunks_us(int64_t m, int64_t n, int64_t k, const lf_lora* lora) {
+  const double chunks = double((m + kDecodeMaxTokens - 1) / kDecodeMaxTokens);
+  if (decode_wide_fits(kDecodeMaxTokens, n, k, lora)) return chunks * wide_us(kDecodeMaxTokens, n, k, lora);
+  if (!lora) return chunks * stream_us(n, k, lora);
+  const double rows = double(lora->num_slices) * lora->max_rank;
+  return chunks * (5.2 + 0.114 * rows + (5.9 + 0.029 * rows) * double(k) / 4096.0 + (6.5 + 0.04 * rows) * double(n) / 4096.0);
+}
+
+// Whether a default call of M > 64 tokens may run on the decode kernels, which
+// contract bf16(code) (relative error about 0.0031 against 0.0024 with the prefill
+// GEMM's exact weights). The line is where these kernels undercut tiles of 256 x
+// 192 at 85 us a round per 4096 of K, by 4 us a round of their own or by the weight
+// bytes: it stays there however fast either becomes, so that a call keeps its
+// precision.
+bool may_decode(int64_t m, int64_t n, int64_t k, const lf_lora* lora) {
+  const int64_t tiles = ((m + 255) / 256) * ((n + 191) / 192);
+  const int64_t cus = device_cus();
+  const double k4 = double(k) / 4096.0;
+  const double tiles_us = double((tiles + cus - 1) / cus) * 85.0 * k4;
+  if (decode_wide_fits(m, n, k, lora) && decode_rounds(m, n) * 4.0 * k4 < tiles_us) return true;
   const int64_t chunks = (m + kDecodeMaxTokens - 1) / kDecodeMaxTokens;
-  return double(chunks) * chunk_us < prefill_us(m, n, k, lora, swiglu);
+  return double(chunks) * stream_us(n, k, lora) < tiles_us + (lora ? 20.0 : 0.0);
 }
 
 // The kernel of a call. Above 8 tokens (2 at N >= 8192, 16 at K > 8192): the wide
 // decode kernel (one launch, base linear with or without LoRA and the SwiGLU
-// output), unless the prefill GEMM is forced or cheaper, or the shape is outside
-// the kernel's range.
+// output) if the shape is in its range; above 64 tokens the fastest of it, the
+// prefill GEMM and decode launches over 64-token chunks (each streams W again but
+// uses every CU, where few tiles leave most of the chip idle), unless a flag names
+// one. (256 tokens x 4096 x 4096 with 128 ragged adapters: wide 61 us, prefill 115
+// us; 256 x 11008: 98 / 67 us; 4096 x 24576 x 64: 911 / 62 us.) Against the faster
+// of decode and prefill over 650 shapes and routings at K >= 1024 the prices lose
+// 0.3 %, over 90 drawn calls of 65..512 tokens with up to 128 adapters 1.8 %.
 int kernel_of(int64_t m, int64_t n, int64_t k, const lf_lora* lora, int32_t flags) {
-  const bool swiglu = (flags & LF_SWIGLU_OUTPUT) != 0;
-  if (decode_wide_fits(m, n, k, lora) && !(flags & LF_PLAN_PREFILL) &&
-      (m <= kDecodeMaxTokens || (flags & LF_PLAN_DECODE_CHUNKS) || wide_cheaper(m, n, k, lora, swiglu)))
-    return LF_KERNEL_DECODE_WIDE;
-  if (m <= kDecodeMaxTokens) return LF_KERNEL_DECODE;
-  if (flags & LF_PLAN_DECODE_CHUNKS) return LF_KERNEL_DECODE_CHUNKS;
-  if (flags & LF_PLAN_PREFILL) return LF_KERNEL_PREFILL;
-  return decode_chunks_cheaper(m, n, k, lora, swiglu) ? LF_KERNEL_DECODE_CHUNKS : LF_KERNEL_PREFILL;
+  const bool wide = decode_wide_fits(m, n, k, lora) && !(flags & LF_PLAN_PREFILL);
+  if (m <= kDecodeMaxTokens) return wide ? LF_KERNEL_DECODE_WIDE : LF_KERNEL_DECODE;
+  if (flags & LF_PLAN_DECODE_CHUNKS) return wide ? LF_KERNEL_DECODE_WIDE : LF_KERNEL_DECODE_CHUNKS;
+  if ((flags & LF_PLAN_PREFILL) || !may_decode(m, n, k, lora)) return LF_KERNEL_PREFILL;
+  const double prefill = prefill_us(m, n, k, lora, (flags & LF_SWIGLU_OUTPUT) != 0);
+  if (wide && wide_us(m, n, k, lora) < prefill) return LF_KERNEL_DECODE_WIDE;
+  return chunks_us(m, n, k, lora) < prefill ? LF_KERNEL_DECODE_CHUNKS : LF_KERNEL_PREFILL;
 }
-
 // Whether lora_apply's two launches over all tokens are cheaper than a launch
 // of the decode kernel's residual form per 64 tokens. Their time grows with
 // the distinct adapters of a tile (500 tokens x 5120 x 4096, 4 adapters: 31 us

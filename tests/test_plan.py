@@ -2,6 +2,7 @@
 
 import ctypes
 import math
+import random
 
 import pytest
 
@@ -42,3 +43,33 @@ def test_refusals():
     for bad in (dict(m=0), dict(n=100), dict(k=0), dict(slices=4), dict(slices=1, rank=65)):
         with pytest.raises(ValueError):
             plan_of(**{**dict(m=128, n=256, k=256), **bad})
+
+
+# Without adapters, and with: calls whose K is short against their tiles' fixed time.
+SHORT = [(2048, 18944, 64, 0), (4096, 24576, 64, 0), (512, 24576, 128, 0), (2048, 8192, 256, 0), (430, 13312, 384, 1), (1024, 24576, 192, 1)]
+
+
+@pytest.mark.parametrize("m,n,k,slices", SHORT)
+def test_short_k_stays_on_the_prefill_gemm(m, n, k, slices):
+    """Its exact weights, and up to twelve times its speed: rounds of decode workgroups have a fixed part."""
+    assert plan_of(m, n, k, slices, 16, 8 * slices).kernel == _lib.LF_KERNEL_PREFILL
+
+
+def _exact_before(m, n, k, slices, rank):
+    """Calls above 64 tokens that are too many, or too long, for the decode kernels by the bound on where
+    they may take a default call: 256 x 192 tiles at 85 us a round per 4096 of K."""
+    rounds = math.ceil(math.ceil(m / 256) * math.ceil(n / 192) / 256)
+    tiles_us = rounds * 85.0 * k / 4096
+    decode_rounds = math.ceil(math.ceil(n / 32 / 8) * 8 * math.ceil(m / 32) / 256)
+    chunks_us = math.ceil(m / 64) * ((6.0 if slices else 0.0) + n * k * 0.5625 / 0.8e6)
+    return decode_rounds * 4.0 * k / 4096 >= tiles_us and chunks_us >= tiles_us + (20.0 if slices else 0.0)
+
+
+def test_no_default_call_leaves_the_exact_weights():
+    rng = random.Random(5)
+    for _ in range(20000):
+        log = lambda lo, hi: math.exp(rng.uniform(math.log(lo), math.log(hi)))
+        m, n, k = int(log(65, 8192)), 64 * max(1, round(log(256, 40000) / 64)), 64 * max(1, round(log(64, 16384) / 64))
+        slices, rank, slots = rng.choice((0, 1, 2, 3)), rng.choice((4, 16, 64)), rng.choice((0, 1, 8, 32, 128))
+        if _exact_before(m, n, k, slices, rank):
+            assert plan_of(m, n, k, slices, rank, slots).kernel == _lib.LF_KERNEL_PREFILL, (m, n, k, slices, rank, slots)
