@@ -74,8 +74,8 @@ struct TilePlan {
 
 // Time of a plan's LoRA call under a routing, us.
 //  - A round's fixed part (start, routes, rounding and stores; without LoRA 5 +
-//    1.2 ri, see tile_plan) and the expand beyond the first slot, per slot and
-//    32-token block.
+//    1.2 ri, see tile_plan) and the expand beyond the first slots: per slot where
+//    a tile rounds once for all, else per slot and 32-token block.
 //  - Producers in the GEMM launch: a unit takes 2 us and, per 4096 of K, 3.7 us
 //    for each 16 A rows and each 64-row pass (four waves, fragment loads). Their
 //    consumers wait for what does not end within the first round's k-loop (2048 x
@@ -87,7 +87,9 @@ double lora_plan_us(const TilePlan& p, double loop, int64_t cus, int64_t k, int 
   const double k4 = double(k) / 4096.0;
   const double rounds = double((p.tiles + cus - 1) / cus);
   const int row_tiles = (slices * max_rank + 15) / 16;
-  const double expand = 1.05 * p.ri * std::max(0.0, r.block - 1.0) * (1.0 + 0.1 * ((max_rank + 15) / 16 - 1));
+  const int steps = (max_rank + 15) / 16;
+  const double expand = p.ri <= kManyRows ? 0.9 * std::max(0.0, r.slots - kFewSlots) * (1.0 + 0.2 * (steps - 1))
+                                          : 1.05 * p.ri * std::max(0.0, r.block - 1.0) * (1.0 + 0.1 * (steps - 1));
   const double gemm = rounds * (loop + 7.5 + 2.25 * p.ri + expand);
   const double serial = std::ceil(r.units / p.zparts);  // units of one producer
   if (!p.z_launch) return 1.02 * gemm + std::max(0.0, serial * (2.0 + 3.7 * k4 * ((row_tiles + 3) / 4 + row_tiles)) - 0.9 * loop);

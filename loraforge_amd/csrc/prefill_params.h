@@ -11,6 +11,10 @@ constexpr int kThreads = 256;
 constexpr int kBM = 256;     // most tokens per tile
 constexpr int kTileN = 256;  // output features per tile
 constexpr int kZSlice = 64;  // zpad columns per slice
+// Tiles of more than kFewSlots slots and at most kManyRows 32-token blocks expand all
+// slots into the accumulators before one rounding pass (gemm_kernel's epilogue).
+constexpr int kFewSlots = 2;
+constexpr int kManyRows = 4;
 
 struct PrefillParams {
   const uint16_t* x;

@@ -1089,79 +1089,193 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(PrefillParams pk) {
       }
     }
     __syncthreads();
-    bool first_ready = true;  // the B of slot 0 requested above is still unused
-    for (int s = 0; s < p.slices; ++s) {
-      const int lo = p.slice_offsets[s];
-      const int hi = p.slice_offsets[s + 1];
-      if (hi <= wn0 || lo >= wn0 + 64) continue;  // this wave's 64 columns miss the slice
-      const bool inside = lo <= wn0 && wn0 + 64 <= hi;
-      const uint4* zs = zs_all + s * kRows * 8;
-      // delta[n][m] = sum_j B_g[n][j] z[m][j], added with the reference's two
-      // roundings to the tokens routed to g and the features of slice s. The
-      // next slot's B is in flight while this slot's MFMAs run.
-      if (!first_ready && nd > 0) request_b(0, bnext);
-      first_ready = false;
-      for (int d = 0; d < nd; ++d) {
+    // The output pair (j, r) of the lane's token in a block: bf16(scale * delta), then the
+    // sum with the rounded base. (token: all ones for a token to update.)
+    auto updated = [&](uint32_t old, float d0, float d1, uint32_t token, bool inside, int lo, int hi, int j, int r) {
+      const uint32_t v = pack_bf16x2(d0, d1);
+      const uint32_t sum = pack_bf16x2(bf16_lo(old) + bf16_lo(v), bf16_hi(old) + bf16_hi(v));
+      uint32_t take = token;
+      if (!inside) {  // columns of other slices keep their value
+        const int n = wn0 + 32 * j + 8 * (r >> 1) + 4 * h + 2 * (r & 1);
+        take &= ((n >= lo && n < hi) ? 0xffffu : 0u) | ((n + 1 >= lo && n + 1 < hi) ? 0xffff0000u : 0u);
+      }
+      return select(take, sum, old);
+    };
+    if (RI <= kManyRows && nd > kFewSlots) {
+      // Tiles of many slots: the deltas of all of a block's slots meet in the idle
+      // accumulators and are rounded once. A slot's MFMAs take the z of its own tokens
+      // and zeros for the others, so a token gets its own slot's sum plus exact zeros.
+      // An infinity or NaN in a slot's B makes NaN of the zeros: a tile that shows one
+      // is done again with a rounding pass per slot. (The masked rounding pass per slot
+      // and block below is 190 VALU instructions. Tokens of 32 slots of rank 16 in turn,
+      // below -> here: 512 x 4096 x 4096 in 64-token tiles 108.5 -> 84.6 us, 512 x 16384
+      // x 1024 in 128-token tiles 144.8 -> 101.3 us. Taller tiles have no registers for
+      // both forms: with both, few slots take 3-12 % longer.)
+      for (int g = -1, d = 0; d < nd; ++d) {
+        if (list[d] == tslot[tid]) g = d;
+        if (d == nd - 1) order[tid] = g;
+      }
+      __syncthreads();
+      int td[RI];         // the lane's token in each block: its slot's place in the list
+      uint64_t left[RI];  // lanes whose slot is still to come
+      auto pick = [&]() {
+        int d = -1;
 #pragma unroll
-        for (int j = 0; j < kJ; ++j)
+        for (int i = RI - 1; i >= 0; --i)
+          if (left[i]) d = __builtin_amdgcn_readlane(td[i], __builtin_ctzll(left[i]));
+        return d;
+      };
+      auto begin = [&]() {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) bq[j][q] = bnext[j][q];
-        if (d + 1 < nd) request_b(d + 1, bnext);
-        const int gd = list[d];
-        const int rank = mrank[d];
-        const int steps = (rank + 15) >> 4;
-        const float scale = mscale[d];
+        for (int i = 0; i < RI; ++i) left[i] = __ballot(td[i] >= 0);
+        return pick();
+      };
 #pragma unroll
-        for (int j = 0; j < kJ; ++j) {
-          // (A rank that fills its last step needs no mask; nor do rows past
-          // N, whose results are never stored.)
-          if (rank & 15) {
-            const int keep = min(mstride[d], rank) - 8 * h;
+      for (int i = 0; i < RI; ++i) td[i] = order[32 * i + c];
+      for (int s = 0; s < p.slices; ++s) {
+        const int lo = p.slice_offsets[s];
+        const int hi = p.slice_offsets[s + 1];
+        if (hi <= wn0 || lo >= wn0 + 64) continue;  // this wave's 64 columns miss the slice
+        const bool inside = lo <= wn0 && wn0 + 64 <= hi;
+        const uint4* zs = zs_all + s * kRows * 8;
+        int d = begin();     // (slot 0, whose B is in flight)
+        bool each = false;   // a rounding pass per slot
+        while (d >= 0) {
+          uint32_t done = 0;  // blocks whose token has its delta
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-              if (q < steps) bq[j][q] = keep_first(bq[j][q], keep - 16 * q);
+          for (int i = 0; i < RI; ++i)
+#pragma unroll
+            for (int j = 0; j < kJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 16; ++r) acc.v[i][j][r] = 0.f;
+          do {
+            const int slot = d;
+            const int rank = mrank[slot];
+            const int keep = min(mstride[slot], rank) - 8 * h;
+            const int steps = (rank + 15) >> 4;
+#pragma unroll
+            for (int j = 0; j < kJ; ++j)
+#pragma unroll
+              for (int q = 0; q < 4; ++q) bq[j][q] = bnext[j][q];
+#pragma unroll
+            for (int i = 0; i < RI; ++i) left[i] &= ~__ballot(td[i] == slot);
+            d = pick();
+            request_b(max(d, 0), bnext);  // (after the last slot, for the next slice)
+            if (rank & 15)
+#pragma unroll
+              for (int j = 0; j < kJ; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                  if (q < steps) bq[j][q] = keep_first(bq[j][q], keep - 16 * q);
+#pragma unroll
+            for (int i = 0; i < RI; ++i) {
+              const bool mine = td[i] == slot;
+              if (__ballot(mine) == 0) continue;  // no token of the slot in this block
+              if (mine) done |= 1u << i;
+#pragma unroll
+              for (int q = 0; q < 4; ++q)
+                if (q < steps) {
+                  uint4 z = zs[swz(32 * i + c, 2 * q + h)];
+                  if (!mine) z = make_uint4(0, 0, 0, 0);
+#pragma unroll
+                  for (int j = 0; j < kJ; ++j) acc.v[i][j] = mfma32(as_bf16x8(bq[j][q]), as_bf16x8(z), acc.v[i][j]);
+                }
+            }
+          } while (d >= 0 && !each);
+          if (!each) {
+            float nan = 0.f;
+#pragma unroll
+            for (int i = 0; i < RI; ++i)
+#pragma unroll
+              for (int j = 0; j < kJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) nan = fmaf(acc.v[i][j][r], 0.f, nan);
+            if (__ballot(nan != nan) != 0) {
+              each = true;
+              d = begin();
+              continue;
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < RI; ++i) {
+            const uint32_t token = (done >> i) & 1 ? 0xffffffffu : 0u;
+            if (__ballot(token != 0) == 0) continue;
+            const float scale = mscale[max(td[i], 0)];
+#pragma unroll
+            for (int j = 0; j < kJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 8; ++r)
+                o.v[i][j][r] = updated(o.v[i][j][r], acc.v[i][j][2 * r] * scale, acc.v[i][j][2 * r + 1] * scale, token, inside, lo, hi, j, r);
           }
         }
-        // 32-token blocks with a token of gd, the delta of one block two
-        // MFMA chains ahead of its use.
-        uint32_t here = 0;
-        bool mine[RI];
-#pragma unroll
-        for (int i = 0; i < RI; ++i) {
-          mine[i] = tslot[32 * i + c] == gd;
-          if (__ballot(mine[i]) != 0) here |= 1u << i;
-        }
-#pragma unroll
-        for (int i = 0; i < RI; ++i) {
-          if (((here >> i) & 1) == 0) continue;
-          f32x16 delta[kJ];
+      }
+    } else {
+      bool first_ready = true;  // the B of slot 0 requested above is still unused
+      for (int s = 0; s < p.slices; ++s) {
+        const int lo = p.slice_offsets[s];
+        const int hi = p.slice_offsets[s + 1];
+        if (hi <= wn0 || lo >= wn0 + 64) continue;  // this wave's 64 columns miss the slice
+        const bool inside = lo <= wn0 && wn0 + 64 <= hi;
+        const uint4* zs = zs_all + s * kRows * 8;
+        // delta[n][m] = sum_j B_g[n][j] z[m][j], added with the reference's two
+        // roundings to the tokens routed to g and the features of slice s. The
+        // next slot's B is in flight while this slot's MFMAs run.
+        if (!first_ready && nd > 0) request_b(0, bnext);
+        first_ready = false;
+        for (int d = 0; d < nd; ++d) {
 #pragma unroll
           for (int j = 0; j < kJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) delta[j][r] = 0.f;
+            for (int q = 0; q < 4; ++q) bq[j][q] = bnext[j][q];
+          if (d + 1 < nd) request_b(d + 1, bnext);
+          const int gd = list[d];
+          const int rank = mrank[d];
+          const int steps = (rank + 15) >> 4;
+          const float scale = mscale[d];
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            if (q < steps) {
-              const bf16x8 z = as_bf16x8(zs[swz(32 * i + c, 2 * q + h)]);
+          for (int j = 0; j < kJ; ++j) {
+            // (A rank that fills its last step needs no mask; nor do rows past
+            // N, whose results are never stored.)
+            if (rank & 15) {
+              const int keep = min(mstride[d], rank) - 8 * h;
 #pragma unroll
-              for (int j = 0; j < kJ; ++j) delta[j] = mfma32(as_bf16x8(bq[j][q]), z, delta[j]);
+              for (int q = 0; q < 4; ++q)
+                if (q < steps) bq[j][q] = keep_first(bq[j][q], keep - 16 * q);
             }
-          // bf16(scale * delta), then the sum with the rounded base; other
-          // slots' tokens and other slices' columns keep their value.
-          const uint32_t token = mine[i] ? 0xffffffffu : 0u;
+          }
+          // 32-token blocks with a token of gd, the delta of one block two
+          // MFMA chains ahead of its use.
+          uint32_t here = 0;
+          bool mine[RI];
 #pragma unroll
-          for (int j = 0; j < kJ; ++j)
+          for (int i = 0; i < RI; ++i) {
+            mine[i] = tslot[32 * i + c] == gd;
+            if (__ballot(mine[i]) != 0) here |= 1u << i;
+          }
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
-              const uint32_t v = pack_bf16x2(delta[j][2 * r] * scale, delta[j][2 * r + 1] * scale);
-              const uint32_t sum = pack_bf16x2(bf16_lo(o.v[i][j][r]) + bf16_lo(v), bf16_hi(o.v[i][j][r]) + bf16_hi(v));
-              uint32_t take = token;
-              if (!inside) {
-                const int n = wn0 + 32 * j + 8 * (r >> 1) + 4 * h + 2 * (r & 1);
-                take &= ((n >= lo && n < hi) ? 0xffffu : 0u) | ((n + 1 >= lo && n + 1 < hi) ? 0xffff0000u : 0u);
+          for (int i = 0; i < RI; ++i) {
+            if (((here >> i) & 1) == 0) continue;
+            f32x16 delta[kJ];
+#pragma unroll
+            for (int j = 0; j < kJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 16; ++r) delta[j][r] = 0.f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              if (q < steps) {
+                const bf16x8 z = as_bf16x8(zs[swz(32 * i + c, 2 * q + h)]);
+#pragma unroll
+                for (int j = 0; j < kJ; ++j) delta[j] = mfma32(as_bf16x8(bq[j][q]), z, delta[j]);
               }
-              o.v[i][j][r] = select(take, sum, o.v[i][j][r]);
-            }
+            // bf16(scale * delta), then the sum with the rounded base; other
+            // slots' tokens and other slices' columns keep their value.
+            const uint32_t token = mine[i] ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int j = 0; j < kJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 8; ++r)
+                o.v[i][j][r] = updated(o.v[i][j][r], delta[j][2 * r] * scale, delta[j][2 * r + 1] * scale, token, inside, lo, hi, j, r);
+          }
         }
       }
     }

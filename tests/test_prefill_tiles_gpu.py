@@ -142,16 +142,35 @@ def test_every_height_with_adapters(swiglu, rows, k, device):
     near(nf4_lora_linear(p.x, p.q, p.st, lora=p.lora, swiglu=swiglu, plan="prefill"), p.expected(True, swiglu))
 
 
-@pytest.mark.parametrize("m,k,rows", [(182, 320, 64), (278, 192, 96), (374, 896, 128), (470, 1088, 160)])
+@pytest.mark.parametrize("m,k,rows,slots", [(182, 320, 64, 12), (278, 192, 96, 12), (374, 896, 128, 12), (470, 1088, 160, 3)])
 @pytest.mark.parametrize("r,slices", [(3, 1), (33, 3), (16, 3)])
-def test_slots_in_turn(m, k, rows, r, slices, device):
-    """Twelve slots in turn among the tokens, slice bounds inside a wave's columns."""
+def test_slots_in_turn(m, k, rows, slots, r, slices, device):
+    """Slots in turn among the tokens, slice bounds inside a wave's columns."""
     n = WIDE_N
-    p = Problem(m, n, k, device, r=r, slots=12, slices=slices, routes="in turn")
+    p = Problem(m, n, k, device, r=r, slots=slots, slices=slices, routes="in turn")
     p.bounds = [0, n] if slices == 1 else [0, n // 3 + 5, n - 70, n]
     p.lora.slice_offsets = torch.tensor(p.bounds, dtype=torch.int32, device=device)
     assert plan_of(m, n, k, p.lora).tile_rows == rows
     near(nf4_lora_linear(p.x, p.q, p.st, lora=p.lora, plan="prefill"), p.expected())
+
+
+@pytest.mark.parametrize("m,rows", [(182, 64), (278, 96), (374, 128), (470, 160)])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), -3.0e38])
+def test_an_infinite_b_reaches_its_own_slot_only(m, rows, value, device):
+    """Slots that share an expand pass multiply each other's B with zeros."""
+    n, k = WIDE_N, 320
+    p = Problem(m, n, k, device, slots=9, routes="in turn")
+    assert plan_of(m, n, k, p.lora).tile_rows == rows
+    good = nf4_lora_linear(p.x, p.q, p.st, lora=p.lora, plan="prefill")
+    bad = p.lora.b_store.clone().reshape(9, n, 16)
+    bad[4, 100:300, 7] = value
+    p.lora.b_store = bad.reshape(-1)
+    y = nf4_lora_linear(p.x, p.q, p.st, lora=p.lora, plan="prefill")
+    own = p.routes == 4
+    assert torch.equal(y[~own], good[~own])
+    assert torch.equal(y[own][:, :100], good[own][:, :100]) and torch.equal(y[own][:, 300:], good[own][:, 300:])
+    changed = y[own][:, 100:300].float()
+    assert not torch.isfinite(changed).any() if value != -3.0e38 else bool((changed.abs() > 1e30).all())
 
 
 @pytest.mark.parametrize("m,n,k,r", [(2048, 8192, 1024, 16), (1024, 16384, 512, 16), (1024, 16384, 1024, 16)])
