@@ -5,16 +5,28 @@
 // HBM-bound: per 64-element block it reads 32 packed bytes + 4 scale bytes
 // and writes 128 bytes. Each lane decodes one packed dword (8 elements) per
 // step and stores 16 bytes, so every load (256 B/wave) and store (1 KiB/wave)
-// instruction is fully coalesced. The stores are non-temporal: the output is
-// four times the packed bytes and larger than the caches can hold back, and
-// writing it through them cost half the rate (24576 x 4096: fp32 scales 55.7
-// -> 37.3 us, 257 MB at 6.9 TB/s; nested 72.5 -> 39.6 us; 8192 x 1024 5.6 ->
-// 4.3 us). Two independent steps per lane (one: 38.4 us, four: 37.7 us at
-// 24576 x 4096); four for a nested state of at least 32 M elements (39.6 us
+// instruction is fully coalesced. How it stores goes by the output's size,
+// so that the product that reads the weight next gains too (of each pair: the
+// call, and the call with the product of 16 tokens behind it, over weights in
+// turn whose packed bytes come from HBM):
+//  - to 96 MiB written through the L2 (`sc1`): the output stays in the
+//    memory-side cache, and no write-back waits for the kernel's end.
+//    2048 x 2048 3.5 and 13.6 us (plain stores 4.1 and 14.2, non-temporal 3.5
+//    and 16.4), 8192 x 1024 6.2 and 16.8 (6.4 and 17.9, 6.1 and 18.5), 4096 x 4096
+//    10.8 and 33.0 (11.3 and 30.4, 11.1 and 35.1), 11008 x 4096 24.4 and 45.0
+//    (25.1 and 45.3, 26.0 and 53.9).
+//  - beyond, where outputs in turn drive each other out of that cache of
+//    256 MiB, non-temporal: 16384 x 4096 of one packed weight into three outputs
+//    25.4 us against 37.8 (11008 x 4096 17.7 against 18.9), 24576 x 4096 nested
+//    38 against 63. Its reader pays for that (24576 x 4096 54 and 97 us against
+//    50 and 84 written through) up to 256 MiB and gains beyond (32832 x 4096 with
+//    256 tokens 150 against 166).
+// Two independent steps per lane (one: 38.4 us, four: 37.7 us at 24576 x 4096
+// with fp32 scales); four for a nested state of at least 32 M elements (39.6 us
 // against 44.7 us: fewer workgroups stage the 256-entry code2), two below
-// (4096 x 4096 7.5 us against 7.7 us). Packed bytes at an address that is not 4-byte
-// aligned, or an output that is not 16-byte aligned (a contiguous view at an
-// odd offset, which the reference accepts), take the same kernel with byte
+// (4096 x 4096 7.5 us against 7.7 us). Packed bytes at an address that is not
+// 4-byte aligned, or an output that is not 16-byte aligned (a contiguous view at
+// an odd offset, which the reference accepts), take the same kernel with byte
 // loads and 2-byte stores.
 #include <chrono>
 #include <mutex>
@@ -28,6 +40,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int64_t kLargeNested = int64_t(32) << 20;  // elements: four steps per lane
+constexpr int64_t kThroughMost = int64_t(48) << 20;  // elements (96 MiB): stores written through
 
 // Packed dword w of the weight (bytes 4w..4w+3, little endian).
 template <bool kAligned>
@@ -41,9 +54,13 @@ __device__ __forceinline__ uint32_t load_packed(const uint8_t* __restrict__ pack
 }
 
 // Elements 8w..8w+7 of the output.
-template <bool kAligned>
-__device__ __forceinline__ void store_elements(uint16_t* __restrict__ out, int64_t w, uint4 v) {
-  if constexpr (kAligned) {
+template <bool kAligned, bool kThrough>
+__device__ __forceinline__ void store_elements(uint16_t* __restrict__ out, int64_t w, int64_t ndwords, uint4 v) {
+  if constexpr (kAligned && kThrough) {
+    constexpr int kSc1 = 16;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, int(16 * ndwords), 0x00027000);
+    __builtin_amdgcn_raw_buffer_store_b128((u32x4){v.x, v.y, v.z, v.w}, rsrc, int(16 * w), 0, kSc1);
+  } else if constexpr (kAligned) {
     __builtin_nontemporal_store((u32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<u32x4*>(out) + w);
   } else {
     uint16_t* p = out + 8 * w;
@@ -80,7 +97,7 @@ __constant__ const float kCanonical[16] = {
 // canonical codebook (word null: unchecked).
 constexpr uint32_t kAnswered = 2;
 
-template <bool kDouble, bool kAligned, int kSteps>
+template <bool kDouble, bool kAligned, int kSteps, bool kThrough>
 __global__ __launch_bounds__(kThreads) void nf4_dequant_kernel(const uint8_t* __restrict__ packed,
                                                                ScaleSource src, const float* __restrict__ code,
                                                                uint16_t* __restrict__ out, int64_t ndwords,
@@ -110,7 +127,7 @@ __global__ __launch_bounds__(kThreads) void nf4_dequant_kernel(const uint8_t* __
     if (w < ndwords) {
       // 8 elements per dword, 64 per block: block = w / 8.
       const float scale = block_scale(src, w >> 3, code2, offset);
-      store_elements<kAligned>(out, w, decode_dword(words[s], scale, table));
+      store_elements<kAligned, kThrough>(out, w, ndwords, decode_dword(words[s], scale, table));
     }
   }
 }
@@ -139,14 +156,20 @@ int launch_dequant(const uint8_t* qweight, const ScaleSource& src, const float* 
   LF_REQUIRE(grid < (int64_t(1) << 31), "tensor too large");
   auto s = static_cast<hipStream_t>(stream);
   const bool vec = aligned16(out) && (reinterpret_cast<uintptr_t>(qweight) & 3u) == 0;
-  if (src.scales) {
-    auto k = vec ? nf4_dequant_kernel<false, true, 2> : nf4_dequant_kernel<false, false, 2>;
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, s, qweight, src, code, out, ndwords, verdict);
-  } else {
-    auto k = steps == 4 ? (vec ? nf4_dequant_kernel<true, true, 4> : nf4_dequant_kernel<true, false, 4>)
-                        : (vec ? nf4_dequant_kernel<true, true, 2> : nf4_dequant_kernel<true, false, 2>);
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, s, qweight, src, code, out, ndwords, verdict);
-  }
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, s, qweight, src, code, out, ndwords, verdict);
+  };
+  const bool through = numel <= kThroughMost;
+  if (src.scales)
+    launch(!vec      ? nf4_dequant_kernel<false, false, 2, false>
+           : through ? nf4_dequant_kernel<false, true, 2, true>
+                     : nf4_dequant_kernel<false, true, 2, false>);
+  else if (steps == 2)  // (less than kThroughMost)
+    launch(vec ? nf4_dequant_kernel<true, true, 2, true> : nf4_dequant_kernel<true, false, 2, false>);
+  else
+    launch(!vec      ? nf4_dequant_kernel<true, false, 4, false>
+           : through ? nf4_dequant_kernel<true, true, 4, true>
+                     : nf4_dequant_kernel<true, true, 4, false>);
   LF_HIP(hipGetLastError());
   return kOk;
 }

@@ -144,3 +144,29 @@ def test_views_at_unaligned_offsets(q_offset, out_offset, device):
     dequantize_nf4_nested(qv, st, out=nested_out)
     torch.cuda.synchronize()
     assert np.array_equal(_bits(nested_out), expect)
+
+
+# A nested state's two steps and four, stores written through and non-temporal ones: the last and the first size of each.
+@pytest.mark.parametrize("shape", [(8128, 4096), (8192, 4096), (12288, 4096), (12352, 4096)])
+def test_stores_at_the_sizes_where_they_change(shape, device):
+    """Each store form, fp32 and nested scales, every element against the recipe in torch; nothing past the end."""
+    n, k = shape
+    gen = torch.Generator(device=device).manual_seed(n)
+    q = torch.randint(0, 256, (n * k // 2,), generator=gen, device=device, dtype=torch.uint8)
+    code = torch.from_numpy(onf4.NF4_CODE).to(device)
+    nested = NestedState(torch.rand(-(-(n * k // 64) // 256), generator=gen, device=device), torch.rand(256, generator=gen, device=device))
+    absmax = torch.randint(0, 256, (n * k // 64,), generator=gen, device=device, dtype=torch.uint8)
+    state = NF4State(absmax, torch.Size(shape), code, torch.bfloat16, offset=torch.tensor(0.25, device=device), state2=nested)
+    scales = prepare_scales(state)
+    nibbles = torch.stack([q >> 4, q & 15], dim=1).reshape(-1, 64)
+    expect = (code[nibbles.int()] * scales[:, None]).bfloat16().reshape(shape)
+    del nibbles
+    backing = torch.full((n * k + 64,), 7.0, dtype=torch.bfloat16, device=device)
+    out = backing[: n * k].view(shape)
+    for name, call in (("fp32", lambda: dequantize_nf4(q, scales, code, shape, out=out)), ("nested", lambda: dequantize_nf4_nested(q, state, out=out))):
+        print(f"[nf4] stores {shape} {name}", flush=True)
+        out.fill_(7.0)
+        call()
+        torch.cuda.synchronize()
+        assert torch.equal(out, expect), name
+        assert bool((backing[n * k :] == 7.0).all()), name
