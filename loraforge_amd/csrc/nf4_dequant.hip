@@ -196,7 +196,9 @@ extern "C" int lf_nf4_dequant_dq_checked(const uint8_t* qweight, const uint8_t* 
     std::lock_guard<std::mutex> guard(lf::g_page_lock);
     if (lf::g_page == nullptr) {
       void* page = nullptr;
-      LF_HIP(hipHostMalloc(&page, lf::VerdictWords::kWords * sizeof(uint32_t), hipHostMallocPortable));
+      // (Coherent: the host polls a word while its kernel runs.)
+      LF_HIP(hipHostMalloc(&page, lf::VerdictWords::kWords * sizeof(uint32_t),
+                           hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
       lf::g_page = static_cast<uint32_t*>(page);
     }
   }
