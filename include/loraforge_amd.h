@@ -269,6 +269,11 @@ int lf_nf4_lora_plan(int64_t m, int64_t n, int64_t k, int32_t num_slices, int32_
 int lf_lora_apply(const uint16_t* x, int64_t m, int64_t x_stride, int64_t n, int64_t k, const lf_lora* lora,
                   uint16_t* y, int64_t y_stride, void* workspace, int64_t workspace_bytes, int32_t flags, void* stream);
 
+/* Whether lf_lora_apply takes the two launches for a call of this size, given a
+ * workspace that holds the z rows of 128 tokens: host arithmetic. */
+int lf_lora_apply_plan(int64_t m, int64_t n, int64_t k, int32_t num_slices, int32_t max_rank, int32_t num_slots,
+                       int32_t* two_launches);
+
 /* Allocation-free variant of lf_nf4_lora_linear. It has no counterpart in
  * the reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid

@@ -157,6 +157,10 @@ _PROTOTYPES = {
         ctypes.c_int,
         [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, ctypes.POINTER(Plan)],
     ),
+    "lf_lora_apply_plan": (
+        ctypes.c_int,
+        [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, ctypes.POINTER(c_int32)],
+    ),
     "lf_nf4_lora_status": (ctypes.c_int, [c_void_p, c_void_p, ctypes.POINTER(c_int32)]),
     "lf_swiglu": (ctypes.c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p]),
 }

@@ -114,18 +114,34 @@ int kernel_of(int64_t m, int64_t n, int64_t k, const lf_lora* lora, int32_t flag
   return chunks_us(m, n, k, lora) < prefill ? LF_KERNEL_DECODE_CHUNKS : LF_KERNEL_PREFILL;
 }
 // Whether lora_apply's two launches over all tokens are cheaper than a launch
-// of the decode kernel's residual form per 64 tokens. Their time grows with
-// the distinct adapters of a tile (500 tokens x 5120 x 4096, 4 adapters: 31 us
-// against 142 us; 382 x 4096 x 1024, 8 adapters: 50 / 53 us; 300 x 1024 x 1024
-// over 32: 110 / 42 us; 300 x 4096 x 4096 over 128: 210 / 82 us), a launch per 64
-// tokens takes 8 us and 8 us more per 4096 x 4096; above 16 adapters (or a
-// pool of unknown size) the latter.
-bool apply_tiles_cheaper(int64_t m, int64_t n, int64_t k, int num_slots) {
-  if (num_slots < 1 || num_slots > 16) return false;
-  const double size = double(n) * double(k) / (4096.0 * 4096.0);
-  const double tiles_us = (14.0 + 4.2 * num_slots) * std::max(1.0, size);
+// of the decode kernel's residual form per 64 tokens. The former's time grows
+// with the distinct adapters of 64 tokens: 500 tokens x 5120 x 4096 over 4
+// adapters 24.6 us against 142 us, but 300 x 1024 x 1024 over 32 110 against 42
+// and 300 x 4096 x 4096 over 128 210 against 82 (above 16 adapters, or a pool of
+// unknown size, a launch per 64 tokens), which takes 8 us and 8 us more per
+// 4096 x 4096. A launch whose blocks run in one round (N to 4096) is faster
+// than that, and both sides are priced closer there (to 10 % on 256 calls of
+// 65..1000 tokens), the adapters of 64 tokens as the mean of those of tokens in
+// runs and in turn: 192 x 4096 x 4096 over 8 adapters of rank 16 21.5 us in
+// launches against 19.2 in runs and 32.2 in turn, 128 tokens over 4 14.6 us
+// against 17.9 and 20.2; from 256 over 8 (28.5 against 19.6 and 33.9) or at rank
+// 64 (39.9 against 23.6 and 46.0) the two launches.
+bool apply_tiles_cheaper(int64_t m, int64_t n, int64_t k, const lf_lora* lora) {
+  const int slots = lora->num_slots;
+  if (slots < 1 || slots > 16) return false;
+  const double k4 = double(k) / 4096.0;
+  const double size = k4 * double(n) / 4096.0;
+  const double tiles_us = (14.0 + 4.2 * slots) * std::max(1.0, size);
   const double launches_us = double((m + kDecodeMaxTokens - 1) / kDecodeMaxTokens) * (8.0 + 8.0 * size);
-  return tiles_us < launches_us;
+  if (tiles_us >= launches_us) return false;
+  if (n % 256 != 0 || n > 4096) return true;
+  const double rows = double(lora->num_slices) * lora->max_rank;
+  const double split = std::max(1.0, double(n) / 1024.0);  // workgroups that share a token's rows of A
+  const double launch_us = 5.5 + rows * (0.11 + 0.02 * k4 * (4.0 - split));
+  const int64_t rest = m % kDecodeMaxTokens;  // (to 32 tokens the narrow kernel)
+  const double live = 1.0 + (slots - 1) * (0.5 + 0.5 * std::min(1.0, double(kDecodeMaxTokens) / double(m)));
+  return 9.5 + k4 + (2.1 + 0.2 * k4) * live + 0.035 * rows * (1.0 + 0.25 * live) <
+         double(m / kDecodeMaxTokens) * launch_us + (rest > 32 ? launch_us : rest > 0 ? 8.8 : 0.0);
 }
 
 // One decode launch of up to 64 tokens: the wide kernel for the batches and
@@ -244,6 +260,22 @@ extern "C" int lf_nf4_lora_plan(int64_t m, int64_t n, int64_t k, int32_t num_sli
   return lf::kOk;
 }
 
+extern "C" int lf_lora_apply_plan(int64_t m, int64_t n, int64_t k, int32_t num_slices, int32_t max_rank, int32_t num_slots,
+                                  int32_t* two_launches) {
+  LF_REQUIRE(two_launches != nullptr, "null pointer argument");
+  LF_REQUIRE(m > 0 && m < (int64_t(1) << 31), "token count out of range");
+  LF_REQUIRE(n > 0 && k > 0 && n % 64 == 0 && k % 64 == 0, "N and K must be positive multiples of 64");
+  LF_REQUIRE(n < (int64_t(1) << 28) && k < (int64_t(1) << 28), "shape too large");
+  LF_REQUIRE(num_slices >= 1 && num_slices <= 3, "num_slices must be in 1..3");
+  LF_REQUIRE(max_rank >= 1 && max_rank <= 64, "max_rank must be in 1..64");
+  lf_lora lora{};
+  lora.num_slices = num_slices;
+  lora.max_rank = max_rank;
+  lora.num_slots = num_slots;
+  *two_launches = m > lf::kDecodeMaxTokens && lf::apply_tiles_cheaper(m, n, k, &lora);
+  return lf::kOk;
+}
+
 extern "C" int lf_nf4_lora_status(const void* workspace, void* stream, int32_t* status) {
   LF_REQUIRE(workspace && status, "null pointer argument");
   auto s = static_cast<hipStream_t>(stream);
@@ -278,7 +310,7 @@ extern "C" int lf_lora_apply(const uint16_t* x, int64_t m, int64_t x_stride, int
   // over all tokens whose z rows the workspace holds. A workspace that holds
   // fewer than 128 tokens' rows takes the launches per 64 tokens below.
   const int64_t fit = m > lf::kDecodeMaxTokens && !withhold && workspace && lf::aligned16(workspace) &&
-                              lf::apply_tiles_cheaper(m, n, k, lora->num_slots)
+                              lf::apply_tiles_cheaper(m, n, k, lora)
                           ? lf::apply_tiles_tokens(workspace_bytes, lora->num_slices)
                           : 0;
   if (fit >= 128) {

@@ -4,10 +4,13 @@ Gate as in ``test_lora_apply_gpu.py``: max abs/rel 2e-2, relative L2 < 0.005,
 rows without an adapter keep their bits.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
+from loraforge_amd import _lib
 from loraforge_amd.ops import lora_apply
 from loraforge_amd.ops.fused import workspace_bytes
 from tests import _cases
@@ -17,17 +20,25 @@ from tests.test_lora_apply_gpu import check, make_case, on_device
 pytestmark = pytest.mark.gpu
 
 
+def two_launches(m, n, k, slices, ranks):
+    two = ctypes.c_int32()
+    _lib.check(_lib.library().lf_lora_apply_plan(m, n, k, slices, max(ranks), len(ranks), ctypes.byref(two)))
+    return bool(two.value)
+
+
 @pytest.mark.parametrize(
-    "m,n,k,slices,bounds,ranks",
+    "m,n,k,slices,bounds,ranks,two",
     [
-        (193, 64, 64, 1, None, (16,)),  # the fewest tokens that take the two launches; the smallest N and K
-        (257, 320, 192, 3, [0, 190, 257, 320], (64, 7, 0, 16)),  # slice bounds inside fragments, a wave past N; a second z tile of one token
-        (330, 576, 320, 2, [0, 300, 576], (2, 4, 8, 17, 48)),  # a last tile of ten tokens
-        (700, 1024, 1024, 1, None, tuple([4, 8, 16, 32] * 4)),  # 16 slots: the most that take the two launches
-        (300, 1024, 256, 1, None, tuple([4, 8, 16, 32] * 16)),  # 64 slots: launches per 64 tokens
+        (128, 64, 64, 1, None, (16,), False),  # the most tokens of the smallest N and K that take launches per 64 tokens,
+        (129, 64, 64, 1, None, (16,), True),  # and the fewest that take the two launches
+        (257, 320, 192, 3, [0, 190, 257, 320], (64, 7, 0, 16), True),  # slice bounds inside fragments, a wave past N; a second z tile of one token
+        (330, 576, 320, 2, [0, 300, 576], (2, 4, 8, 17, 48), True),  # a last tile of ten tokens
+        (700, 1024, 1024, 1, None, tuple([4, 8, 16, 32] * 4), True),  # 16 slots: the most that take the two launches
+        (300, 1024, 256, 1, None, tuple([4, 8, 16, 32] * 16), False),  # 64 slots: launches per 64 tokens
     ],
 )
-def test_tiles(m, n, k, slices, bounds, ranks, device):
+def test_tiles(m, n, k, slices, bounds, ranks, two, device):
+    assert two_launches(m, n, k, slices, ranks) == two
     case = make_case(m, n, k, ranks, slices=slices, bounds=bounds, seed=m + k)
     x, y, batch = on_device(case, device)
     assert lora_apply(x, y, batch) is y
@@ -46,6 +57,7 @@ def test_routes_in_segments_and_a_workspace_of_few_tokens(device):
     (same bits), one that holds fewer than 128 the launches per 64 tokens (the oracle's gate)."""
     m, n, k = 500, 512, 256
     routes = np.repeat(np.array([2, 0, -1, 1], np.int32), [130, 200, 50, 120])
+    assert two_launches(m, n, k, 1, (32, 16, 8))
     case = make_case(m, n, k, (32, 16, 8), seed=77, routes=routes)
     x, y, batch = on_device(case, device)
     lora_apply(x, y, batch)
@@ -70,6 +82,7 @@ def test_routes_in_segments_and_a_workspace_of_few_tokens(device):
 )
 def test_z_stages(m, n, k, slices, bounds, ranks, device):
     """K where the waves of a z unit have different numbers of stages, and reuse their slots."""
+    assert two_launches(m, n, k, slices, ranks)
     routes = np.arange(m, dtype=np.int32) % (len(ranks) + 1) - 1 if len(ranks) > 1 else np.zeros(m, np.int32)
     case = make_case(m, n, k, ranks, slices=slices, bounds=bounds, seed=m + k, routes=routes)
     x, y, batch = on_device(case, device)

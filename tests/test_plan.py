@@ -73,3 +73,31 @@ def test_no_default_call_leaves_the_exact_weights():
         slices, rank, slots = rng.choice((0, 1, 2, 3)), rng.choice((4, 16, 64)), rng.choice((0, 1, 8, 32, 128))
         if _exact_before(m, n, k, slices, rank):
             assert plan_of(m, n, k, slices, rank, slots).kernel == _lib.LF_KERNEL_PREFILL, (m, n, k, slices, rank, slots)
+
+
+def two_launches(m, n, k, slices, rank, slots):
+    two = ctypes.c_int32()
+    _lib.check(_lib.library().lf_lora_apply_plan(m, n, k, slices, rank, slots, ctypes.byref(two)))
+    return bool(two.value)
+
+
+# Launches of the decode kernel that run in one round of workgroups: faster than the two launches over all tokens up to
+# these sizes, by tokens in turn and by the mean of tokens in turn and in runs.
+@pytest.mark.parametrize(
+    "m,n,k,slices,rank,slots,two",
+    [
+        (65, 4096, 4096, 1, 16, 1, True), (65, 4096, 4096, 1, 16, 4, False), (65, 2048, 8192, 1, 16, 4, False),
+        (128, 4096, 4096, 1, 16, 4, False), (128, 2048, 8192, 1, 16, 4, False), (128, 4096, 4096, 1, 64, 4, True),
+        (192, 4096, 4096, 1, 16, 4, True), (192, 4096, 4096, 1, 16, 8, False), (192, 2048, 8192, 1, 16, 8, False),
+        (192, 4096, 4096, 1, 64, 8, True), (256, 4096, 4096, 1, 16, 8, True), (500, 5120, 4096, 3, 16, 4, True),
+        (64, 4096, 4096, 1, 16, 4, False), (500, 4096, 4096, 1, 16, 17, False),
+    ],
+)
+def test_lora_apply_launches(m, n, k, slices, rank, slots, two):
+    assert two_launches(m, n, k, slices, rank, slots) == two
+
+
+def test_lora_apply_plan_refusals():
+    for bad in (dict(m=0), dict(n=100), dict(k=0), dict(slices=0), dict(slices=4), dict(rank=65)):
+        with pytest.raises(ValueError):
+            two_launches(**{**dict(m=128, n=256, k=256, slices=1, rank=16, slots=4), **bad})
