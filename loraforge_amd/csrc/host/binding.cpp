@@ -10,7 +10,7 @@
 //
 // An eager call of the fused linear spent 29 us on the host in about fifty
 // small Python checks and ctypes conversions, twice the time of a decode
-// kernel at 4096 x 4096; this path takes about 5 us.
+// kernel at 4096 x 4096; this path takes 6 us.
 //
 // The library's entry points are handed over as addresses (init), so this
 // module binds to whatever build of the library the process loaded.

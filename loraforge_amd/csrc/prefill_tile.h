@@ -376,10 +376,11 @@ __device__ __forceinline__ void copy_x(const PrefillParams& p, const XLane& xl, 
 // M-tile mt routed to live slots are sorted by slot (counting sort in LDS)
 // and cut into units of up to 16 tokens of one slot; producer (mt, q) takes
 // units q, q + zparts, ... For a unit it contracts just those tokens with the
-// slices * r rows of A_g, 64 rows (four 16-row tiles) per pass: the eight
+// slices * r rows of A_g, 64 rows (four 16-row tiles) per pass: the four
 // waves take interleaved 32-wide k steps (v_mfma_f32_16x16x32_bf16, A rows as
 // the A operand, the tokens' x as the B operand, four steps of loads in
-// flight), the partial tiles meet in LDS in a fixed order, and
+// flight; in a launch of their own eight waves, 16 rows a pass and whole row
+// pieces through LDS, below), the partial tiles meet in LDS in a fixed order, and
 // z = bf16(x A_g^T) is stored in the slice-padded layout zpad[t][s * 64 + j]
 // (zeros for r <= j < 64). Finally the producer sets its flag
 // zflags[mt * zparts + q] to the call's tag. Work follows the routed tokens:
@@ -626,7 +627,8 @@ __device__ __forceinline__ void produce_z(const PrefillParams& p, int mt, int q,
 // at device scope would invalidate the whole L2 of the XCD under the other
 // workgroups' feet. Each wait is bounded (about a quarter second); a
 // producer that has not set its flag by then has its units recomputed here
-// (same arithmetic, so the same z bits), the status word records it, and the
+// (the sums of a producer in this launch, so its z bits; one of a launch of its
+// own sums over eight waves, another order), the status word records it, and the
 // tile's slot metadata, whose LDS the recomputation borrowed, is reloaded.
 // Returns whether it recomputed anything.
 __device__ bool wait_z(const PrefillParams& p, int mt, uint32_t tag, int* tslot, int* list, int* order, int* mrank,
@@ -725,6 +727,7 @@ __device__ __forceinline__ int tile_row(const PrefillParams& p, int nt, int r) {
 // epoch on) to the GEMM launch, which finds every flag set.
 // (Eight waves: their 128 KiB of copies in flight fill the CU.)
 constexpr int kZThreads = 512;
+#ifdef LF_PREFILL_Z_KERNEL
 __global__ __launch_bounds__(kZThreads) void z_kernel(PrefillParams p) {
   __shared__ __attribute__((aligned(256))) char ring[kZThreads / 64 * 2 * kZSlot];
   __shared__ __attribute__((aligned(16))) float red[kZThreads / 64 * 16 * 17];
@@ -734,6 +737,7 @@ __global__ __launch_bounds__(kZThreads) void z_kernel(PrefillParams p) {
   const int unit = blockIdx.x / p.zrow_parts;
   produce_z<0, 1, kZThreads>(p, unit / p.zparts, unit % p.zparts, blockIdx.x % p.zrow_parts, p.zrow_parts, tag, tslot, list, order, cnt, ustart, red, ring);
 }
+#endif
 
 // Block ids below zblocks (LoRA launches whose last round has room for them)
 // produce the tiles' z rows; the others are GEMM tiles, M-tile b % mtiles on

@@ -99,7 +99,7 @@ def apply_nf4_lora(x, qweight, state, info, table, *, bias=None, out=None, token
 
 
 def apply_lora(x, y, info, table, *, token_slots=None, slice_offsets=None):
-    """``y += LoRA(x)`` in place for SGLang's batch, one launch per 64 tokens.
+    """``y += LoRA(x)`` in place for SGLang's batch: one launch per 64 tokens or two over all of them.
 
     For projections whose base output SGLang computes itself (unquantised
     layers): the Fleet backend's A pass then B pass over ``batch_info``

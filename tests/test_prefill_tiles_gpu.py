@@ -14,6 +14,7 @@ import torch
 
 from loraforge_amd import _lib
 from loraforge_amd.ops import LoraBatch, dequantize_nf4, nf4_lora_linear, quantize_nf4
+from loraforge_amd.ops.fused import _lora_struct, _weight_struct, workspace_bytes
 from tests import _cases
 from tests.test_fused_gpu import bits, close, to_device, workspace_clean
 
@@ -180,3 +181,25 @@ def test_producers_in_a_launch_of_their_own(m, n, k, r, device):
     assert plan_of(m, n, k, p.lora).z_launch == 1
     near(nf4_lora_linear(p.x, p.q, p.st, lora=p.lora, plan="prefill"), p.expected())
     workspace_clean(device)
+
+
+@pytest.mark.parametrize("slices", [1, 3])
+def test_withheld_producers_of_a_launch_of_their_own(slices, device):
+    """No flag is ever set: the GEMM launch's bounded waits run out and its tiles recompute every z row."""
+    m, n, k = 1024, 16384, 256
+    p = Problem(m, n, k, device, slices=slices)
+    assert plan_of(m, n, k, p.lora).z_launch == 1
+    weight, keep = _weight_struct(p.q, p.st, None, n, k, device, m)
+    lora = _lora_struct(p.lora, m, k, n, device)
+    need = workspace_bytes(m, n, k, num_slices=slices, max_rank=p.r)
+    ws = torch.zeros(need, dtype=torch.uint8, device=device)
+    lib, stream = _lib.library(), _lib.stream_of(device)
+    for withhold in (0, _lib.LF_TEST_WITHHOLD_PARTIALS):
+        y = torch.zeros(m, n, dtype=torch.bfloat16, device=device)
+        _lib.check(lib.lf_nf4_lora_linear(p.x.data_ptr(), m, k, weight, None, lora, y.data_ptr(), n, ws.data_ptr(), need,
+                                          _lib.LF_PLAN_PREFILL | withhold, stream))
+        status = ctypes.c_int32(-1)
+        _lib.check(lib.lf_nf4_lora_status(ws.data_ptr(), stream, ctypes.byref(status)))
+        assert status.value == (1 if withhold else 0)
+        near(y, p.expected())
+    del keep

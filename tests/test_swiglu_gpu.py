@@ -199,8 +199,7 @@ def test_fused_swiglu_above_64_tokens_on_both_plans(m, plan, device):
 
 def test_prefill_swiglu_c5_scale(device):
     """The prefill GEMM with the activation in its epilogue at M = 2048 over c5's weight read as
-    a merged gate/up projection (N = 11008: 5504 activation columns, 58 column tiles, the last
-    partial), double quant, 8 segments of rank 32 over the gate/up slices: bit-identical to the
+    a merged gate/up projection (N = 11008: 5504 activation columns, 43 column tiles of 128), double quant, 8 segments of rank 32 over the gate/up slices: bit-identical to the
     linear followed by silu_mul."""
     m, inter, k, rank, segs = 2048, 5504, 4096, 32, 8
     g = torch.Generator(device="cpu").manual_seed(736)
