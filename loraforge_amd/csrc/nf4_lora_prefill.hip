@@ -45,21 +45,21 @@ struct TileCost {
 constexpr TileCost kTileCosts[] = {{8, 75.0}, {6, 60.0}, {5, 57.0}, {4, 53.0}, {3, 52.0}, {2, 41.5}};
 
 // How a tile of `tokens` tokens may be routed over a pool of adapters: slots
-// among its tokens and among 32 of them, and z units (16 tokens of one slot,
-// half a unit lost to each slot). The host does not know the routes, so a plan
+// among its tokens and among 32 of them, and z units (16 tokens of one slot, or
+// 32: half a unit lost to each slot). The host does not know the routes, so a plan
 // is priced for two of them: each slot's tokens together (prompts one after the
 // other), and all slots in turn, the less likely the more tokens a slot has.
 struct Routing {
-  double slots, block, units;
+  double tokens, slots, block, units, units32;
 };
-double units_of(double tokens, double slots) { return std::max(slots, tokens / 16.0 + slots / 2.0); }
+double units_of(double tokens, double slots, double size) { return std::max(slots, tokens / size + slots / 2.0); }
 Routing together(double tokens, double m, double pool) {
   const double slots = std::min({pool, tokens, tokens * pool / m + 1.0});
-  return {slots, 1.0 + std::min(slots - 1.0, 32.0 * pool / m), units_of(tokens, slots)};
+  return {tokens, slots, 1.0 + std::min(slots - 1.0, 32.0 * pool / m), units_of(tokens, slots, 16.0), units_of(tokens, slots, 32.0)};
 }
 Routing in_turn(double tokens, double pool) {
   const double slots = pool * tokens / (pool + tokens);
-  return {slots, pool * 32.0 / (pool + 32.0), units_of(tokens, slots)};
+  return {tokens, slots, pool * 32.0 / (pool + 32.0), units_of(tokens, slots, 16.0), units_of(tokens, slots, 32.0)};
 }
 double in_turn_weight(double m, double pool) { return std::min(0.4, 17.0 * pool / m); }
 constexpr int kPoolUnknown = 16;  // adapters of a call that does not say
@@ -77,11 +77,12 @@ struct TilePlan {
 //    1.2 ri, see tile_plan) and the expand beyond the first slots: per slot where
 //    a tile rounds once for all, else per slot and 32-token block.
 //  - Producers in the GEMM launch: a unit takes 2 us and, per 4096 of K, 3.7 us
-//    for each 16 A rows and each 64-row pass (four waves, fragment loads). Their
-//    consumers wait for what does not end within the first round's k-loop (2048 x
-//    11008 x 4096, two slices of rank 32, SwiGLU: 33 producers in the slack of
-//    192-token tiles 244 us, 168 in that of 256-token tiles 219 us; three slices
-//    of rank 64: 408 / 217 us); their loads cost the first tiles about 2 %.
+//    for each 16 A rows and, in each 64-row pass, for each 16 tokens (four waves,
+//    fragment loads); units of 32 tokens where those of 16 outnumber the producers.
+//    Their consumers wait for what does not end within the first round's k-loop
+//    (2048 x 11008 x 4096, three slices of rank 64: 33 producers in the slack of
+//    192-token tiles 408 us, 168 in that of 256-token tiles 217 us); their loads
+//    cost the first tiles about 2 %.
 //  - In a launch of their own (through LDS, one 16-row pass at a time).
 double lora_plan_us(const TilePlan& p, double loop, int64_t cus, int64_t k, int slices, int max_rank, const Routing& r) {
   const double k4 = double(k) / 4096.0;
@@ -91,8 +92,15 @@ double lora_plan_us(const TilePlan& p, double loop, int64_t cus, int64_t k, int 
   const double expand = p.ri <= kManyRows ? 0.9 * std::max(0.0, r.slots - kFewSlots) * (1.0 + 0.2 * (steps - 1))
                                           : 1.05 * p.ri * std::max(0.0, r.block - 1.0) * (1.0 + 0.1 * (steps - 1));
   const double gemm = rounds * (loop + 7.5 + 2.25 * p.ri + expand);
+  if (!p.z_launch) {
+    const bool pairs = r.units > p.zparts;
+    const int x_tiles = pairs && r.tokens > 16.0 * r.units32 ? 2 : 1;
+    const double each = 2.0 + 3.7 * k4 * ((row_tiles + 3) / 4 * x_tiles + row_tiles);
+    // (Units of 32 are few: of the tiles' different numbers the larger ones count.)
+    const double serial = pairs ? std::max(1.0, r.units32 / p.zparts + 0.6) : std::ceil(r.units / p.zparts);
+    return 1.02 * gemm + std::max(0.0, serial * each - 0.9 * loop);
+  }
   const double serial = std::ceil(r.units / p.zparts);  // units of one producer
-  if (!p.z_launch) return 1.02 * gemm + std::max(0.0, serial * (2.0 + 3.7 * k4 * ((row_tiles + 3) / 4 + row_tiles)) - 0.9 * loop);
   const int parts = z_row_parts(slices, max_rank);
   const double groups = double(p.mtiles * p.zparts * parts);
   const double busy = std::min<double>(r.units, p.zparts) * double(p.mtiles * parts) / double(cus) + 1.0;

@@ -125,7 +125,7 @@ constexpr int kJ = 2;          // 32-feature fragments per wave
 constexpr int kBK = 128;       // k per stage: two NF4 blocks
 constexpr int kXRow = 256;     // bytes of one x row in a stage
 constexpr int kSteps = 8;      // MFMA steps per stage (8 k of each block)
-constexpr int kMinRing = 20 * 1024;  // the z producers' partial tiles
+constexpr int kMinRing = 36 * 1024;  // the z producers' partial tiles
 
 // x stages in LDS: as many as fit beside the packed weights and the LoRA tables.
 template <int RI>
@@ -374,7 +374,8 @@ __device__ __forceinline__ void copy_x(const PrefillParams& p, const XLane& xl, 
 
 // z producers: the launch's first mtiles * zparts workgroups. The tokens of
 // M-tile mt routed to live slots are sorted by slot (counting sort in LDS)
-// and cut into units of up to 16 tokens of one slot; producer (mt, q) takes
+// and cut into units of up to 16 tokens of one slot (of 32 where the launch has
+// fewer producers than that makes units: see produce_units); producer (mt, q) takes
 // units q, q + zparts, ... For a unit it contracts just those tokens with the
 // slices * r rows of A_g, 64 rows (four 16-row tiles) per pass: the four
 // waves take interleaved 32-wide k steps (v_mfma_f32_16x16x32_bf16, A rows as
@@ -470,10 +471,14 @@ __device__ __forceinline__ f32x4 contract_staged(const PrefillParams& p, const u
 // (contract_staged). kRowTiles: 16-row tiles of A per pass; parts: workgroups that
 // share a unit's rows (this one takes the passes rp, rp + parts, ...). In the
 // producers' own launch through LDS, one tile a pass, up to four workgroups a
-// unit. In the GEMM launch 4 steps of four tiles (its registers hold no more
-// beside the output tile).
+// unit. In the GEMM launch 4 steps of four tiles (8 steps: slower by 10 %, the
+// address unit takes 64 cycles for each fragment load whatever is in flight).
+// That bounds a unit (64 A rows of 4096: 20 us), so where a producer has several,
+// they take 32 tokens: the A fragments are loaded once for two x fragments. 2048 x
+// 11008 x 4096 in 192-token tiles with three producers each, two slices of rank 32,
+// SwiGLU: 238 -> 210 us (222 in 256-token tiles with 21; no adapters 186).
 template <int kUnitSteps, int kRowTiles, int kThreads = prefill::kThreads>
-__device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int parts, int* tslot, int* list, int* order, int* cnt,
+__device__ __forceinline__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int parts, int* tslot, int* list, int* order, int* cnt,
                               int* ustart, float* red, char* ring = nullptr) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -516,6 +521,15 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
     }
   }
   __syncthreads();
+  // (Every producer of the tile, and a consumer that recomputes, finds the same size.)
+  constexpr int kTokTiles = kUnitSteps == 0 ? 1 : 2;
+  int size = kUnit;
+  if constexpr (kTokTiles == 2) {
+    int units = 0;
+    for (int d = 0; d < nd; ++d) units += (cnt[d] + kUnit - 1) / kUnit;
+    if (units > p.zparts) size = 2 * kUnit;
+    __syncthreads();
+  }
   if (tid == 0) {
     int pos = 0, units = 0;
     for (int d = 0; d < nd; ++d) {
@@ -523,7 +537,7 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
       cnt[d] = pos;       // first position of slot d's tokens in `order`
       ustart[d] = units;  // first unit of slot d
       pos += n;
-      units += (n + kUnit - 1) / kUnit;
+      units += (n + size - 1) / size;
     }
     cnt[nd] = pos;
     ustart[nd] = units;
@@ -536,8 +550,8 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
   for (int u = rp == 0 ? q : units; u < units; u += p.zparts) {
     int d = 0;
     while (ustart[d + 1] <= u) ++d;
-    const int first = cnt[d] + (u - ustart[d]) * kUnit;
-    const int ntok = min(kUnit, cnt[d + 1] - first);
+    const int first = cnt[d] + (u - ustart[d]) * size;
+    const int ntok = min(size, cnt[d + 1] - first);
     const int r = p.ranks[list[d]];
     for (int i = tid; i < ntok * zw; i += kThreads) {
       const int t = i / zw;
@@ -548,28 +562,35 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
   for (int u = q; u < units; u += p.zparts) {
     int d = 0;
     while (ustart[d + 1] <= u) ++d;
-    const int first = cnt[d] + (u - ustart[d]) * kUnit;
-    const int ntok = min(kUnit, cnt[d + 1] - first);
+    const int first = cnt[d] + (u - ustart[d]) * size;
+    const int ntok = min(size, cnt[d + 1] - first);
     const int gd = list[d];
     const int r = p.ranks[gd];
     const int rows = p.slices * r;
     const uint16_t* abase = p.a_store + p.a_offsets[gd];
-    const int tok = m0 + order[first + min(c, ntok - 1)];
-    const uint16_t* xrow = p.x + int64_t(tok) * p.x_stride + 8 * kg;
-    for (int j0 = rp * kPassRows; j0 < rows; j0 += parts * kPassRows) {
-      f32x4 acc[kRowTiles];
+    const uint16_t* xrow[kTokTiles];
 #pragma unroll
-      for (int jt = 0; jt < kRowTiles; ++jt) acc[jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < kTokTiles; ++i)
+      xrow[i] = p.x + int64_t(m0 + order[first + min(16 * i + c, ntok - 1)]) * p.x_stride + 8 * kg;
+    const bool two = ntok > kUnit;  // (uniform)
+    for (int j0 = rp * kPassRows; j0 < rows; j0 += parts * kPassRows) {
+      f32x4 acc[kTokTiles][kRowTiles];
+#pragma unroll
+      for (int i = 0; i < kTokTiles; ++i)
+#pragma unroll
+        for (int jt = 0; jt < kRowTiles; ++jt) acc[i][jt] = (f32x4){0.f, 0.f, 0.f, 0.f};
       const int tiles = (min(kPassRows, rows - j0) + 15) >> 4;  // uniform
       if constexpr (kUnitSteps == 0) {
-        acc[0] = contract_staged<kWaves>(p, abase, j0, rows, m0, order + first, ntok, ring);
+        acc[0][0] = contract_staged<kWaves>(p, abase, j0, rows, m0, order + first, ntok, ring);
       } else for (int s0 = wave; s0 < steps; s0 += kWaves * kUnitSteps) {
         // Loads of this batch's steps first (past the end: a readable step, not contracted).
-        uint4 xb[kUnitSteps], ab[kUnitSteps][kRowTiles];
+        uint4 xb[kUnitSteps][kTokTiles], ab[kUnitSteps][kRowTiles];
 #pragma unroll
         for (int v = 0; v < kUnitSteps; ++v) {
           const int st = min(s0 + v * kWaves, steps - 1);
-          xb[v] = *reinterpret_cast<const uint4*>(xrow + st * 32);
+#pragma unroll
+          for (int i = 0; i < kTokTiles; ++i)
+            if (i == 0 || two) xb[v][i] = *reinterpret_cast<const uint4*>(xrow[i] + st * 32);
 #pragma unroll
           for (int jt = 0; jt < kRowTiles; ++jt)
             if (jt < tiles)
@@ -581,22 +602,29 @@ __device__ void produce_units(const PrefillParams& p, int mt, int q, int rp, int
           if (s0 + v * kWaves < steps)
 #pragma unroll
             for (int jt = 0; jt < kRowTiles; ++jt)
-              if (jt < tiles) acc[jt] = mfma16(as_bf16x8(ab[v][jt]), as_bf16x8(xb[v]), acc[jt]);
+              if (jt < tiles)
+#pragma unroll
+                for (int i = 0; i < kTokTiles; ++i)
+                  if (i == 0 || two) acc[i][jt] = mfma16(as_bf16x8(ab[v][jt]), as_bf16x8(xb[v][i]), acc[i][jt]);
       }
-      // acc[jt][e] = this wave's partial of z[token c][A row j0 + 16 jt + 4 kg + e].
+      // acc[i][jt][e] = this wave's partial of z[token 16 i + c][A row j0 + 16 jt + 4 kg + e].
+      constexpr int kRedRow = 16 * kTokTiles + 1;
 #pragma unroll
-      for (int jt = 0; jt < kRowTiles; ++jt)
+      for (int i = 0; i < kTokTiles; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) red[((wave * kRowTiles + jt) * 16 + 4 * kg + e) * 17 + c] = acc[jt][e];
+        for (int jt = 0; jt < kRowTiles; ++jt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) red[((wave * kRowTiles + jt) * 16 + 4 * kg + e) * kRedRow + 16 * i + c] = acc[i][jt][e];
+      static_assert(kUnitSteps == 0 || kWaves * kRowTiles * 16 * kRedRow * 4 <= kMinRing, "the partial tiles fit the idle x ring");
       __syncthreads();
-      for (int o = tid; o < kPassRows * kUnit; o += kThreads) {
-        const int jr = o >> 4;  // A row within the pass
-        const int t = o & 15;
+      for (int o = tid; o < kPassRows * kUnit * kTokTiles; o += kThreads) {
+        const int jr = o / (kUnit * kTokTiles);  // A row within the pass
+        const int t = o % (kUnit * kTokTiles);
         const int j = j0 + jr;
         if (t < ntok && j < rows) {
           float sum = 0.f;
 #pragma unroll
-          for (int w = 0; w < kWaves; ++w) sum += red[((w * kRowTiles + (jr >> 4)) * 16 + (jr & 15)) * 17 + t];
+          for (int w = 0; w < kWaves; ++w) sum += red[((w * kRowTiles + (jr >> 4)) * 16 + (jr & 15)) * kRedRow + t];
           const int sl = j / r;
           store_z(p.zpad + int64_t(m0 + order[first + t]) * zw + sl * kZSlice + (j - sl * r), uint16_t(f32_to_bf16(sum)));
         }
@@ -649,8 +677,10 @@ __device__ bool wait_z(const PrefillParams& p, int mt, uint32_t tag, int* tslot,
   const uint64_t lost = uint64_t(missing[0]) | (uint64_t(missing[1]) << 32);
   if (lost == 0) return false;
   if (threadIdx.x == 0) __hip_atomic_store(p.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // (Producers of a launch of their own cut other units: then all are made again. One tile in
+  // flight, fewer registers: the sums are the same.)
   for (int q = 0; q < p.zparts; ++q)
-    if ((lost >> q) & 1) produce_units<4, 4>(p, mt, q, 0, 1, tslot, list, order, mrank, mstride, red);
+    if (p.zblocks == 0 || ((lost >> q) & 1)) produce_units<1, 1>(p, mt, q, 0, 1, tslot, list, order, mrank, mstride, red);
   int tid = threadIdx.x;
   tie(tid);  // (opaque: nothing of this rare path is kept from before the k-loop)
   for (int d = tid; d < list[kMaxList]; d += kThreads) {

@@ -28,11 +28,15 @@ def test_z_producers_keep_up_with_the_tiles(m, n, k, slices, rank, swiglu):
     plan = plan_of(m, n, k, slices, rank, 8, _lib.LF_PLAN_PREFILL | (_lib.LF_SWIGLU_OUTPUT if swiglu else 0))
     if plan.z_launch:
         return
-    units = math.ceil(plan.tile_rows / 16 + 0.5 * (1 + 8 * plan.tile_rows / m))
+    size = 16
+    units = math.ceil(plan.tile_rows / size + 0.5 * (1 + 8 * plan.tile_rows / m))
+    if units > plan.z_parts:  # then they are of 32 tokens
+        size = 32
+        units = math.ceil(plan.tile_rows / size + 0.5 * (1 + 8 * plan.tile_rows / m))
     row_tiles = math.ceil(slices * rank / 16)
-    # A unit takes 3.7 us per 4096 of K for each 16 A rows and each pass of 64 of them, the k-loop 10 us per
-    # 32 tokens (and no less than 47 us, for the decode of the weights).
-    z_us = math.ceil(units / plan.z_parts) * 3.7 * (math.ceil(row_tiles / 4) + row_tiles)
+    # A unit takes 3.7 us per 4096 of K for each 16 A rows and, in each pass of 64 of them, for each 16 tokens, the
+    # k-loop 10 us per 32 tokens (and no less than 47 us, for the decode of the weights).
+    z_us = math.ceil(units / plan.z_parts) * 3.7 * (math.ceil(row_tiles / 4) * size / 16 + row_tiles)
     loop_us = max(47.0, 10.0 * plan.tile_rows / 32)
     tiles = math.ceil(m / plan.tile_rows) * math.ceil(n / 256)
     share = 0.2 if row_tiles <= 4 else 0.9

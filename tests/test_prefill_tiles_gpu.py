@@ -183,17 +183,25 @@ def test_producers_in_a_launch_of_their_own(m, n, k, r, device):
     workspace_clean(device)
 
 
-@pytest.mark.parametrize("slices", [1, 3])
-def test_withheld_producers_of_a_launch_of_their_own(slices, device):
-    """No flag is ever set: the GEMM launch's bounded waits run out and its tiles recompute every z row."""
-    m, n, k = 1024, 16384, 256
-    p = Problem(m, n, k, device, slices=slices)
-    assert plan_of(m, n, k, p.lora).z_launch == 1
+# Producers in a launch of their own; and in the GEMM launch, fewer than a tile has units of 16 tokens, so of 32.
+WITHHELD = [(1024, 16384, 256, 1, 16, True), (1024, 16384, 256, 3, 16, True), (700, 5120, 1088, 1, 16, False),
+            (1350, 4096, 576, 3, 33, False), (2048, 5120, 320, 2, 33, False)]
+
+
+@pytest.mark.parametrize("routes", ["together", "in turn"])
+@pytest.mark.parametrize("m,n,k,slices,r,launch", WITHHELD)
+def test_producers_and_their_recomputation(m, n, k, slices, r, launch, routes, device):
+    """Without flags the GEMM launch's bounded waits run out and its tiles recompute every z row: the same
+    bits where the producers are in that launch."""
+    p = Problem(m, n, k, device, slices=slices, r=r, routes=routes)
+    plan = plan_of(m, n, k, p.lora)
+    assert plan.z_launch == launch and (launch or plan.z_parts < plan.tile_rows // 16)
     weight, keep = _weight_struct(p.q, p.st, None, n, k, device, m)
     lora = _lora_struct(p.lora, m, k, n, device)
-    need = workspace_bytes(m, n, k, num_slices=slices, max_rank=p.r)
+    need = workspace_bytes(m, n, k, num_slices=slices, max_rank=r)
     ws = torch.zeros(need, dtype=torch.uint8, device=device)
     lib, stream = _lib.library(), _lib.stream_of(device)
+    out = []
     for withhold in (0, _lib.LF_TEST_WITHHOLD_PARTIALS):
         y = torch.zeros(m, n, dtype=torch.bfloat16, device=device)
         _lib.check(lib.lf_nf4_lora_linear(p.x.data_ptr(), m, k, weight, None, lora, y.data_ptr(), n, ws.data_ptr(), need,
@@ -202,4 +210,6 @@ def test_withheld_producers_of_a_launch_of_their_own(slices, device):
         _lib.check(lib.lf_nf4_lora_status(ws.data_ptr(), stream, ctypes.byref(status)))
         assert status.value == (1 if withhold else 0)
         near(y, p.expected())
+        out.append(y)
+    assert launch or torch.equal(*out)
     del keep
