@@ -9,7 +9,7 @@
 // its fp32 block scales rebuilt into the workspace, and z may have a launch of
 // its own (nf4_lora_prefill.hip):
 //  - z producers: z = bf16(x A_g^T) of just the tokens routed to g (gathered,
-//    16 at a time, MFMA), into a slice-padded workspace zpad[m][s*64 + j] (zeros
+//    16 or 32 at a time, MFMA), into a slice-padded workspace zpad[m][s*64 + j] (zeros
 //    past r); then the producer's flag is set to the call's tag (call_epoch.h).
 //  - GEMM tiles of 32 RI tokens x 256 output features, four waves, one per
 //    SIMD with up to 512 registers: a wave owns all the tile's tokens x 64
